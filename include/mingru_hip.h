@@ -314,6 +314,41 @@ int mg_delta_gated_bwd(const void* Q, const void* K, const void* V, const void* 
                        int dk, int dv, int chunk, int dtype, void* ws, size_t ws_bytes,
                        mg_stream_t stream);
 
+/* ---- elementwise scans on bf16 tensors --------------------------------------------
+ * The scans above with bf16 tensors (void*), computed in fp32.  No reference
+ * kernels: the reference casts to fp32 around its fp32 kernels
+ * (src/mingru/triton_scans.py:1233-1290).  Workspaces as the fp32 forms.  `state`
+ * (mg_*_state_bytes, fp32) receives the forward's fp32 states at every sub-chunk
+ * start, from which the backward restarts; the forward takes NULL when no backward
+ * follows.  mg_log_scan_bf16_* use mg_log_scan_state_bytes. */
+size_t mg_linear_scan_bf16_state_bytes(int64_t B, int64_t T, int64_t D);
+int mg_linear_scan_bf16_fwd(const void* a, const void* b, void* A, void* Bc, float* state,
+                            int64_t B, int64_t T, int64_t D, void* ws, size_t ws_bytes,
+                            mg_stream_t stream);
+int mg_linear_scan_bf16_bwd(const void* a, const void* b, const float* state, const void* gA,
+                            const void* gB, void* da, void* db, int64_t B, int64_t T, int64_t D,
+                            void* ws, size_t ws_bytes, mg_stream_t stream);
+int mg_log_scan_bf16_fwd(const void* lc, const void* lv, void* h, float* hstate, int64_t B,
+                         int64_t T, int64_t D, void* ws, size_t ws_bytes, mg_stream_t stream);
+int mg_log_scan_bf16_bwd(const void* lc, const void* lv, const float* hstate, const void* gh,
+                         void* dlc, void* dlv, int64_t B, int64_t T, int64_t D, void* ws,
+                         size_t ws_bytes, mg_stream_t stream);
+/* The fused gate scans: kind 0 SignedMinGRU (p0, p1, p2 = s, z, hpre), 1 coupled, 2
+ * MinGRU (p0, p1 = k, hpre; p2, d2 unused; h0 = log h0).  p* and d* rows lie `ld` (>= D)
+ * elements apart; h0 (B,D) is bf16 (h0_half = 1) or fp32; dt (B,T) and lam (D) are given
+ * together (time decay) or both NULL; dlam and ddt as mg_signed_gate_scan_decay_bwd,
+ * each may be NULL; dh0 is fp32. */
+size_t mg_gate_scan_bf16_state_bytes(int64_t B, int64_t T, int64_t D);
+int mg_gate_scan_bf16_fwd(int kind, const void* p0, const void* p1, const void* p2, int64_t ld,
+                          const void* h0, int h0_half, const float* dt, const float* lam, void* h,
+                          float* state, int64_t B, int64_t T, int64_t D, void* ws,
+                          size_t ws_bytes, mg_stream_t stream);
+int mg_gate_scan_bf16_bwd(int kind, const void* p0, const void* p1, const void* p2, int64_t ld,
+                          const float* dt, const float* lam, const float* state, const void* gh,
+                          void* d0, void* d1, void* d2, float* dh0, float* dlam, float* ddt,
+                          int64_t B, int64_t T, int64_t D, void* ws, size_t ws_bytes,
+                          mg_stream_t stream);
+
 /* ---- streaming decode: one recurrent step (inference) -----------------------------
  * No reference kernels: these replace the eager bodies of the mixers' step()
  * (src/mingru/min_gru.py:1399-1448 MinGRU, SignedMinGRU.step, 3611-3688

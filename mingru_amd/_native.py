@@ -48,6 +48,18 @@ _SIGNATURES = {
     "mg_mingru_gate_scan_workspace_bytes": (_SZ, [_I64, _I64, _I64]),
     "mg_mingru_gate_scan_fwd": (_I32, [_P] * 4 + [_I64, _I64, _I64, _P, _SZ, _P]),
     "mg_mingru_gate_scan_bwd": (_I32, [_P] * 8 + [_I64, _I64, _I64, _P, _SZ, _P]),
+    "mg_linear_scan_bf16_state_bytes": (_SZ, [_I64, _I64, _I64]),
+    "mg_linear_scan_bf16_fwd": (_I32, [_P] * 5 + [_I64, _I64, _I64, _P, _SZ, _P]),
+    "mg_linear_scan_bf16_bwd": (_I32, [_P] * 7 + [_I64, _I64, _I64, _P, _SZ, _P]),
+    "mg_log_scan_bf16_fwd": (_I32, [_P] * 4 + [_I64, _I64, _I64, _P, _SZ, _P]),
+    "mg_log_scan_bf16_bwd": (_I32, [_P] * 6 + [_I64, _I64, _I64, _P, _SZ, _P]),
+    "mg_gate_scan_bf16_state_bytes": (_SZ, [_I64, _I64, _I64]),
+    "mg_gate_scan_bf16_fwd": (
+        _I32, [_I32] + [_P] * 3 + [_I64, _P, _I32] + [_P] * 4 + [_I64, _I64, _I64, _P, _SZ, _P],
+    ),
+    "mg_gate_scan_bf16_bwd": (
+        _I32, [_I32] + [_P] * 3 + [_I64] + [_P] * 10 + [_I64, _I64, _I64, _P, _SZ, _P],
+    ),
     "mg_gate_step": (_I32, [_I32] + [_P] * 6 + [_I64, _P]),
     "mg_delta_step": (_I32, [_P] * 8 + [_I64, _I32, _I32, _I32, _P]),
     "mg_log_scan_state_bytes": (_SZ, [_I64, _I64, _I64]),

@@ -39,11 +39,14 @@ HIPCC_FLAGS = [
 ]
 
 
-# Per-source extra flags.  scan_elementwise.hip issues its header atomics from one
-# thread; LLVM's atomic optimizer would turn each into a wave reduction that waits
-# for the atomic's result at once, ahead of the chunk loads it should overlap.
+# Per-source extra flags.  The elementwise scans (mg_elementwise.h) issue their header
+# atomics from one thread; LLVM's atomic optimizer would turn each into a wave
+# reduction that waits for the atomic's result at once, ahead of the chunk loads it
+# should overlap.
+_ONE_THREAD_ATOMICS = ["-mllvm", "-amdgpu-atomic-optimizer-strategy=None"]
 EXTRA_FLAGS = {
-    "scan_elementwise.hip": ["-mllvm", "-amdgpu-atomic-optimizer-strategy=None"],
+    "scan_elementwise.hip": _ONE_THREAD_ATOMICS,
+    "scan_elementwise_bf16.hip": _ONE_THREAD_ATOMICS,
 }
 
 

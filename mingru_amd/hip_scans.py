@@ -357,6 +357,49 @@ class _LinearScanFn(torch.autograd.Function):
         return da.to(ctx.out_dtype), db.to(ctx.out_dtype)
 
 
+def _bf16_rows(*ts: torch.Tensor):
+    """Contiguous, 16-byte aligned bf16 inputs for the bf16 kernels."""
+    return [_contig(t, torch.bfloat16) for t in ts]
+
+
+def _all_bf16(*ts: torch.Tensor) -> bool:
+    return all(t.dtype == torch.bfloat16 for t in ts)
+
+
+class _LinearScanBf16Fn(torch.autograd.Function):
+    """bf16 ``a``, ``b``: read and written as bf16, computed in fp32; the backward restarts
+    from the fp32 states the forward records."""
+
+    @staticmethod
+    def forward(ctx, a, b):
+        a16, b16 = _bf16_rows(a, b)
+        Bn, T, D = a16.shape
+        A, Bc = torch.empty_like(a16), torch.empty_like(a16)
+        state = None
+        if any(ctx.needs_input_grad):
+            state = torch.empty(_size("mg_linear_scan_bf16_state_bytes", Bn, T, D) // 4,
+                                dtype=torch.float32, device=a16.device)
+        ws = _scan_workspace(_size("mg_linear_scan_workspace_bytes", Bn, T, D), a16.device)
+        _call("mg_linear_scan_bf16_fwd", _ptr(a16), _ptr(b16), _ptr(A), _ptr(Bc), _ptr(state),
+              Bn, T, D, _ptr(ws), ws.numel(), _stream(a16))
+        _check_workspace(ws, a16)
+        ctx.save_for_backward(a16, b16, state)
+        return A, Bc
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, gA, gB):
+        a16, b16, state = ctx.saved_tensors
+        Bn, T, D = a16.shape
+        gA16, gB16 = _bf16_rows(gA, gB)
+        da, db = torch.empty_like(a16), torch.empty_like(a16)
+        ws = _scan_workspace(_size("mg_linear_scan_workspace_bytes", Bn, T, D), a16.device)
+        _call("mg_linear_scan_bf16_bwd", _ptr(a16), _ptr(b16), _ptr(state), _ptr(gA16),
+              _ptr(gB16), _ptr(da), _ptr(db), Bn, T, D, _ptr(ws), ws.numel(), _stream(a16))
+        _check_workspace(ws, a16)
+        return da, db
+
+
 def _linear_scan_impl(a: torch.Tensor, b: torch.Tensor):
     """``SCAN_IMPLS['linear_scan']``: same contract as the eager ``linear_scan``."""
     if a.ndim != 3 or b.ndim != 3 or a.shape != b.shape:
@@ -367,7 +410,8 @@ def _linear_scan_impl(a: torch.Tensor, b: torch.Tensor):
     _same_device(a, b)
     if a.numel() == 0:
         return a.new_empty(a.shape), b.new_empty(b.shape)
-    return _funnel("linear_scan", _LinearScanFn.apply, a, b)
+    fn = _LinearScanBf16Fn if _all_bf16(a, b) else _LinearScanFn
+    return _funnel("linear_scan", fn.apply, a, b)
 
 
 # ---------------------------------------------------------------------------
@@ -446,6 +490,58 @@ class _SignedGateScanFn(torch.autograd.Function):
         return ds.to(od), dz.to(od), dhp.to(od), dh0.to(od), g_dt, g_lam, None
 
 
+class _GateScanBf16Fn(torch.autograd.Function):
+    """The fused gate scans on bf16 pre-activations ``p0, p1, p2`` (``p2`` is None for the
+    MinGRU gates): read and written as bf16, computed in fp32; the backward restarts from
+    the fp32 states the forward records.  ``h0`` keeps its own type, bf16 or fp32."""
+
+    @staticmethod
+    def forward(ctx, p0, p1, p2, h0, dt, lam, kind):
+        q0, q1 = _bf16_rows(p0, p1)
+        q2 = None if p2 is None else _bf16_rows(p2)[0]
+        half = h0.dtype == torch.bfloat16
+        h0c = _contig(h0, torch.bfloat16) if half else _as_f32(h0)[0]
+        Bn, T, D = q0.shape
+        h = torch.empty_like(q0)
+        dt32, lam32 = (None, None) if dt is None else _decay_args(dt, lam, q0)
+        state = None
+        if any(ctx.needs_input_grad):
+            state = torch.empty(_size("mg_gate_scan_bf16_state_bytes", Bn, T, D) // 4,
+                                dtype=torch.float32, device=q0.device)
+        ws = _scan_workspace(_size("mg_signed_gate_scan_workspace_bytes", Bn, T, D), q0.device)
+        _call("mg_gate_scan_bf16_fwd", kind, _ptr(q0), _ptr(q1), _ptr(q2), D, _ptr(h0c),
+              int(half), _ptr(dt32), _ptr(lam32), _ptr(h), _ptr(state), Bn, T, D, _ptr(ws),
+              ws.numel(), _stream(q0))
+        _check_workspace(ws, q0)
+        ctx.save_for_backward(q0, q1, q2, state, dt32, lam32)
+        ctx.kind = kind
+        ctx.dtypes = (None if dt is None else dt.dtype, None if lam is None else lam.dtype)
+        return h
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, gh):
+        q0, q1, q2, state, dt32, lam32 = ctx.saved_tensors
+        Bn, T, D = q0.shape
+        (gh16,) = _bf16_rows(gh)
+        d0, d1 = torch.empty_like(q0), torch.empty_like(q0)
+        d2 = None if q2 is None else torch.empty_like(q0)
+        dh0 = torch.empty(Bn, 1, D, dtype=torch.float32, device=q0.device)
+        dlam = ddt = None
+        if dt32 is not None:
+            need = ctx.needs_input_grad
+            dlam, ddt = _decay_partials((Bn, T, D), need[5], need[4], q0.device)
+        ws = _scan_workspace(_size("mg_signed_gate_scan_workspace_bytes", Bn, T, D), q0.device)
+        _call("mg_gate_scan_bf16_bwd", ctx.kind, _ptr(q0), _ptr(q1), _ptr(q2), D, _ptr(dt32),
+              _ptr(lam32), _ptr(state), _ptr(gh16), _ptr(d0), _ptr(d1), _ptr(d2), _ptr(dh0),
+              _ptr(dlam), _ptr(ddt), Bn, T, D, _ptr(ws), ws.numel(), _stream(q0))
+        _check_workspace(ws, q0)
+        dtd, lamd = ctx.dtypes
+        g_dt = ddt.sum(0).to(dtd) if ddt is not None else None
+        g_lam = dlam.sum(0).to(lamd) if dlam is not None else None
+        return d0, d1, d2, dh0.to(d0.dtype), g_dt, g_lam, None
+
+
 def _check_decay(what: str, like: torch.Tensor, dt, lam) -> None:
     if (dt is None) != (lam is None):
         raise ScanFallback(f"{what}: dt and lam must be given together")
@@ -489,6 +585,9 @@ def signed_gate_scan_impl(s: torch.Tensor, z: torch.Tensor, hpre: torch.Tensor,
     _check_decay("signed gate scan", s, dt, lam)
     if s.numel() == 0:
         return s.new_empty(s.shape)
+    if _all_bf16(s, z, hpre):
+        return _funnel("signed gate scan", _GateScanBf16Fn.apply, s, z, hpre, h0, dt, lam,
+                       GATE_STEP_KINDS["signed_coupled" if coupled else "signed"])
     return _funnel("signed gate scan", _SignedGateScanFn.apply, s, z, hpre, h0, dt, lam,
                    bool(coupled))
 
@@ -574,6 +673,9 @@ def mingru_gate_scan_impl(k: torch.Tensor, hpre: torch.Tensor, log_h0: torch.Ten
     _check_decay("MinGRU gate scan", k, dt, lam)
     if k.numel() == 0:
         return k.new_empty(k.shape)
+    if _all_bf16(k, hpre):
+        return _funnel("MinGRU gate scan", _GateScanBf16Fn.apply, k, hpre, None, log_h0, dt, lam,
+                       GATE_STEP_KINDS["mingru"])
     return _funnel("MinGRU gate scan", _MinGRUGateScanFn.apply, k, hpre, log_h0, dt, lam)
 
 
@@ -618,6 +720,40 @@ class _LogScanFn(torch.autograd.Function):
         return dlc.to(ctx.out_dtype), dlv.to(ctx.out_dtype)
 
 
+class _LogScanBf16Fn(torch.autograd.Function):
+    """bf16 ``log_coeffs``, ``log_values``: read and written as bf16, computed in the
+    extended range; the backward restarts from the recorded states."""
+
+    @staticmethod
+    def forward(ctx, log_coeffs, log_values):
+        lc, lv = _bf16_rows(log_coeffs, log_values)
+        Bn, T, D = lc.shape
+        h = torch.empty_like(lc)
+        hstate = None
+        if any(ctx.needs_input_grad):
+            hstate = torch.empty(_size("mg_log_scan_state_bytes", Bn, T, D) // 4,
+                                 dtype=torch.float32, device=lc.device)
+        ws = _scan_workspace(_size("mg_log_scan_workspace_bytes", Bn, T, D), lc.device)
+        _call("mg_log_scan_bf16_fwd", _ptr(lc), _ptr(lv), _ptr(h), _ptr(hstate), Bn, T, D,
+              _ptr(ws), ws.numel(), _stream(lc))
+        _check_workspace(ws, lc)
+        ctx.save_for_backward(lc, lv, hstate)
+        return h
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, gh):
+        lc, lv, hstate = ctx.saved_tensors
+        Bn, T, D = lc.shape
+        (gh16,) = _bf16_rows(gh)
+        dlc, dlv = torch.empty_like(lc), torch.empty_like(lv)
+        ws = _scan_workspace(_size("mg_log_scan_workspace_bytes", Bn, T, D), lc.device)
+        _call("mg_log_scan_bf16_bwd", _ptr(lc), _ptr(lv), _ptr(hstate), _ptr(gh16), _ptr(dlc),
+              _ptr(dlv), Bn, T, D, _ptr(ws), ws.numel(), _stream(lc))
+        _check_workspace(ws, lc)
+        return dlc, dlv
+
+
 def _parallel_scan_log_impl(log_coeffs: torch.Tensor, log_values: torch.Tensor):
     """``SCAN_IMPLS['parallel_scan_log']``: same contract as the eager op."""
     if (
@@ -634,7 +770,8 @@ def _parallel_scan_log_impl(log_coeffs: torch.Tensor, log_values: torch.Tensor):
     _same_device(log_coeffs, log_values)
     if log_coeffs.numel() == 0:
         return log_coeffs.new_empty(log_coeffs.shape)
-    return _funnel("parallel_scan_log", _LogScanFn.apply, log_coeffs, log_values)
+    fn = _LogScanBf16Fn if _all_bf16(log_coeffs, log_values) else _LogScanFn
+    return _funnel("parallel_scan_log", fn.apply, log_coeffs, log_values)
 
 
 # ---------------------------------------------------------------------------
