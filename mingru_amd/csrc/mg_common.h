@@ -136,10 +136,9 @@ __device__ __forceinline__ unsigned mg_next_ticket(unsigned* header, unsigned ep
 // workgroup, as in the one-ticket form.
 // UNIFORM marks the ticket and epoch, which every lane reads from the same LDS
 // words, as wave-uniform (mg_uniform), so that what the body derives from them
-// (chunk, lane group, row bases) stays in scalar registers.  It is a per-kernel
-// choice: it frees vector registers where a kernel is at the cap (the linear
-// backward: 38 spilled registers -> 5), and it was slower by 1-2% in kernels that
-// are not.
+// (chunk, lane group, row bases) stays in scalar registers.  The elementwise scans set
+// it; the block-matrix backward, far from the register cap, was slower with it (217 ->
+// 220 us at B=16, T=4096, n=256).
 template <bool UNIFORM = false, typename Body>
 __device__ __forceinline__ void mg_persistent(unsigned* header, unsigned chunks, Body&& body) {
   __shared__ unsigned s_ticket, s_epoch;
@@ -163,14 +162,14 @@ __device__ __forceinline__ void mg_persistent(unsigned* header, unsigned chunks,
   }
 }
 
-// Workgroups of kernel `k` (blocks of `threads`) the current device holds at once,
-// the grid of a persistent launch.  Cached per (kernel, device, block) in a fixed
+// Workgroups of kernel `k` (blocks of `threads`) the current device holds at once, at
+// most `max_per_cu` on a CU: the grid of a persistent launch.  Cached per (kernel, device, block) in a fixed
 // table: no allocation, so allocation-free entry points may call it.
-inline unsigned mg_resident(const void* k, int threads) {
+inline unsigned mg_resident(const void* k, int threads, unsigned max_per_cu = ~0u) {
   struct Entry {
     const void* k;
     int dev, threads;
-    unsigned n;
+    unsigned per, cus;
   };
   constexpr int CAP = 256;
   static Entry cache[CAP];
@@ -180,16 +179,16 @@ inline unsigned mg_resident(const void* k, int threads) {
   if (hipGetDevice(&dev) != hipSuccess) dev = 0;
   std::lock_guard<std::mutex> lock(mu);
   for (int i = 0; i < used; ++i)
-    if (cache[i].k == k && cache[i].dev == dev && cache[i].threads == threads) return cache[i].n;
+    if (cache[i].k == k && cache[i].dev == dev && cache[i].threads == threads)
+      return (cache[i].per < max_per_cu ? cache[i].per : max_per_cu) * cache[i].cus;
   int per = 0, cus = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, threads, 0) != hipSuccess || per < 1)
     per = 1;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
       cus < 1)
     cus = 1;
-  const unsigned n = (unsigned)per * (unsigned)cus;
-  if (used < CAP) cache[used++] = Entry{k, dev, threads, n};
-  return n;
+  if (used < CAP) cache[used++] = Entry{k, dev, threads, (unsigned)per, (unsigned)cus};
+  return ((unsigned)per < max_per_cu ? (unsigned)per : max_per_cu) * (unsigned)cus;
 }
 
 __device__ __forceinline__ void mg_slot_put(mg_slot_t* p, float v, unsigned epoch) {

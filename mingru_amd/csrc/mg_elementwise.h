@@ -55,6 +55,12 @@ constexpr int GATE_TSUB_BWD = 4;
 constexpr int GATE_TSUB_FWD_NARROW = 8;
 // Workgroups a launch needs before it runs 4 columns per lane: one per CU.
 constexpr int64_t EW_FILL_WGS = 256;
+// Workgroups per CU of a look-back launch.  More in flight only lengthen the walks over
+// predecessors that have no inclusive prefix yet: linear_scan forward / backward at
+// B=3, T=1000, D=2047 (1 column per lane) takes 36 / 51 us with 1, 41 / 58 with 2 and
+// 57 / 58 with 4; the log scans of bf16 rows (2, 4096, 771) want 2 (44 / 53 against
+// 48 / 62 us with 1).
+constexpr unsigned EW_MAX_PER_CU = 2;
 
 // Launch forms of the chunked scans.  EW_LOOKBACK is one launch whose
 // workgroups combine chunk carries by decoupled look-back.  A small problem
@@ -655,20 +661,30 @@ struct EwThread {
   bool valid;  // false only for a ticket beyond the grid (workspace protocol broken)
   int64_t col;
   bool col_ok;
+  unsigned cl;   // the columns the lane loads: its own, or the row's last where it has none
+  int64_t b0;    // first row of the batch row, batch * T
+  // The row to load for step t: t, or the last one past the sequence end.  Loads are
+  // issued unconditionally -- a load under a condition became a branch of its own, with
+  // a wait for the register it replaced -- and a step past the end is made neutral where
+  // its value matters.  (linear_scan forward at (16, 4096, 1024) 184 -> 176 us, the
+  // MinGRU gates 186 -> 142 us, the signed gates 195 -> 182 us.)
+  __device__ __forceinline__ int64_t row(int64_t t, int64_t T) const {
+    return b0 + (t < T ? t : T - 1);
+  }
 };
 
 // The thread's chunk, lane group and columns for ticket `ticket` of the launch:
 // the (lane group, chunk) pair ticket % n_lg, ticket / n_lg (chunks from the end
-// for a REVERSE scan).
-// UNI: the wave index is marked wave-uniform as well (see mg_persistent's UNIFORM).
-template <int VEC, bool REVERSE, bool UNI = false>
+// for a REVERSE scan).  The ticket and the wave index are wave-uniform, so row
+// addresses stay in scalar registers and a load takes one 32-bit column offset.
+template <int VEC, bool REVERSE>
 __device__ __forceinline__ EwThread ew_thread_at(const EwGeom& g, unsigned ticket,
                                                  unsigned long long epoch) {
   EwThread th;
   th.valid = true;
   th.epoch = epoch;
   th.lane = threadIdx.x & (MG_WAVE - 1);
-  th.w = UNI ? (int)mg_uniform(threadIdx.x / MG_WAVE) : (int)(threadIdx.x / MG_WAVE);
+  th.w = (int)mg_uniform(threadIdx.x / MG_WAVE);
   int k = (int)(ticket / (unsigned)g.n_lg);
   th.lg = (int)(ticket - (unsigned)k * (unsigned)g.n_lg);
   th.c = REVERSE ? g.n_chunks - 1 - k : k;
@@ -676,19 +692,78 @@ __device__ __forceinline__ EwThread ew_thread_at(const EwGeom& g, unsigned ticke
   int tile = th.lg - th.bb * g.n_tiles;
   th.col = (int64_t)tile * (MG_WAVE * VEC) + th.lane * VEC;
   th.col_ok = th.col < g.D;
+  th.cl = (unsigned)(th.col_ok ? th.col : g.D - VEC);
+  th.b0 = (int64_t)th.bb * g.T;
   return th;
 }
+
+// Element offsets of the rows a wave loads, th.row(t0), th.row(t0 + 1), ..., times ld:
+// one scalar add a row instead of a 64-bit product.
+struct EwRows {
+  int64_t off, ld, left;
+  __device__ __forceinline__ EwRows(const EwThread& th, int64_t t0, int64_t T, int64_t ld_)
+      : off(th.row(t0, T) * ld_), ld(ld_), left(T - 1 - t0) {}
+  __device__ __forceinline__ int64_t next() {
+    const int64_t o = off;
+    off += left > 0 ? ld : 0;
+    --left;
+    return o;
+  }
+};
 
 // Runs body(ticket, epoch) for the chunks of this workgroup: with the look-back
 // (PH = EW_LOOKBACK) a persistent workgroup takes tickets until they run out
 // (mg_persistent); the two-launch forms take one chunk per workgroup, in
 // workgroup order, since no workgroup waits on another.
-template <int PH, bool UNI = false, typename Body>
+template <int PH, typename Body>
 __device__ __forceinline__ void ew_chunks(const EwGeom& g, unsigned* header, Body&& body) {
   if constexpr (PH == EW_LOOKBACK) {
-    mg_persistent<UNI>(header, (unsigned)g.n_lg * (unsigned)g.n_chunks, body);
+    mg_persistent<true>(header, (unsigned)g.n_lg * (unsigned)g.n_chunks, body);
   } else {
     body(blockIdx.x, PH == EW_AGG ? ew_agg_begin(header) : 0ull);
+  }
+}
+
+// Persistent workgroups (mg_persistent's protocol) with two row buffers, for the kernels
+// whose rows fit twice (linear_scan forward, the gate scans on bf16): load(ticket,
+// rows) issues a chunk's loads, finish(ticket, epoch, rows, mid) runs the chunk and calls
+// mid() in every thread once its local aggregates are formed.  There the next ticket is
+// shared, and its rows load while this chunk's carry and outputs run.  With one buffer a
+// CU's single workgroup loaded, scanned and stored in turn: the signed gates on bf16
+// (16, 4096, 1024) took 196 us forward and 337 backward, as long as on fp32 at twice
+// the bytes; with two, and the loads of a chunk free of branches, 126 and 234 us.
+template <typename Rows, typename Load, typename Finish>
+__device__ __forceinline__ void ew_persistent2(const EwGeom& g, unsigned* header, Load&& load,
+                                               Finish&& finish) {
+  __shared__ unsigned s_ticket, s_epoch;
+  const unsigned chunks = (unsigned)g.n_lg * (unsigned)g.n_chunks;
+  if (threadIdx.x == 0) {
+    const unsigned e0 =
+        __hip_atomic_load(header + MG_H_EPOCH, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+    s_ticket = mg_next_ticket(header, e0, chunks);
+    s_epoch = e0;
+  }
+  __syncthreads();
+  unsigned t = mg_uniform(s_ticket);
+  const unsigned e = mg_uniform(s_epoch);
+  Rows r0, r1;
+  if (t < chunks) load(t, r0);
+  auto step = [&](unsigned tk, Rows& r, Rows& nr) {
+    unsigned next = 0u;
+    if (threadIdx.x == 0) next = mg_next_ticket(header, e, chunks);
+    unsigned tn = 0u;
+    finish(tk, e, r, [&] {
+      if (threadIdx.x == 0) s_ticket = next;
+      __syncthreads();
+      tn = mg_uniform(s_ticket);
+      if (tn < chunks) load(tn, nr);
+    });
+    return tn;
+  };
+  while (t < chunks) {
+    t = step(t, r0, r1);
+    if (t >= chunks) break;
+    t = step(t, r1, r0);
   }
 }
 
@@ -708,27 +783,27 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void ew_fwd_kernel(
   constexpr bool NT = PH != EW_REDUCE;
   constexpr bool HALF = !std::is_same_v<E, float>;
   static_assert(!HALF || TSUB % LIN_STATE == 0, "recorded states at whole sub-chunks");
-  using Rows = Raw<E, VEC>[TSUB];
+  using Row = Raw<E, VEC>[TSUB];
+  struct Rows {
+    Row a, b;
+  };
   const int64_t T = g.T, D = g.D;
-  // The thread's TSUB rows of a and b for ticket `ticket` (identity past the end).
-  auto load = [&](unsigned ticket, Rows& av, Rows& bv) {
+  // The thread's TSUB rows of a and b for ticket `ticket`.  Steps past the end need no
+  // care: nothing follows them.
+  auto load = [&](unsigned ticket, Row& av, Row& bv) {
     const EwThread th = ew_thread_at<VEC, false>(g, ticket, 0u);
     const int64_t t0 = (int64_t)th.c * (WAVES * TSUB) + th.w * TSUB;
+    EwRows rows(th, t0, T, D);
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
-      const int64_t t = t0 + s;
-      if (th.col_ok && t < T) {
-        load_raw<VEC, NT>(av[s], x0 + (th.bb * T + t) * D + th.col);
-        load_raw<VEC, NT>(bv[s], x1 + (th.bb * T + t) * D + th.col);
-      } else {
-        av[s].fill(1.f);
-        bv[s].fill(0.f);
-      }
+      const int64_t off = rows.next();
+      load_raw<VEC, NT>(av[s], x0 + off + th.cl);
+      load_raw<VEC, NT>(bv[s], x1 + off + th.cl);
     }
   };
   // The chunk from its rows: local aggregates, then `mid` (run by every thread),
   // then the carry and the outputs.
-  auto finish = [&](unsigned ticket, unsigned long long epoch, Rows& av, Rows& bv, auto&& mid) {
+  auto finish = [&](unsigned ticket, unsigned long long epoch, Row& av, Row& bv, auto&& mid) {
     const EwThread th = ew_thread_at<VEC, false>(g, ticket, epoch);
     const int64_t t0 = (int64_t)th.c * (WAVES * TSUB) + th.w * TSUB;
     Aff<1> loc[VEC], seed[VEC], carry[VEC];
@@ -783,43 +858,13 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void ew_fwd_kernel(
   };
   if constexpr (PH != EW_LOOKBACK) {
     const unsigned long long tag = PH == EW_AGG ? ew_agg_begin(header) : 0ull;
-    Rows av, bv;
+    Row av, bv;
     load(blockIdx.x, av, bv);
     finish(blockIdx.x, tag, av, bv, [] {});
   } else {
-    // Persistent workgroups (mg_persistent's protocol) with two row buffers: the
-    // next ticket is shared once this chunk's local aggregates are formed, and its
-    // rows load while this chunk's carry and outputs run.
-    __shared__ unsigned s_ticket, s_epoch;
-    const unsigned chunks = (unsigned)g.n_lg * (unsigned)g.n_chunks;
-    if (threadIdx.x == 0) {
-      const unsigned e0 =
-          __hip_atomic_load(header + MG_H_EPOCH, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
-      s_ticket = mg_next_ticket(header, e0, chunks);
-      s_epoch = e0;
-    }
-    __syncthreads();
-    unsigned t = s_ticket;
-    const unsigned e = s_epoch;
-    Rows a0, b0, a1, b1;
-    if (t < chunks) load(t, a0, b0);
-    auto step = [&](unsigned tk, Rows& av, Rows& bv, Rows& nav, Rows& nbv) {
-      unsigned next = 0u;
-      if (threadIdx.x == 0) next = mg_next_ticket(header, e, chunks);
-      unsigned tn = 0u;
-      finish(tk, e, av, bv, [&] {
-        if (threadIdx.x == 0) s_ticket = next;
-        __syncthreads();
-        tn = s_ticket;
-        if (tn < chunks) load(tn, nav, nbv);
-      });
-      return tn;
-    };
-    while (t < chunks) {
-      t = step(t, a0, b0, a1, b1);
-      if (t >= chunks) break;
-      t = step(t, a1, b1, a0, b0);
-    }
+    ew_persistent2<Rows>(
+        g, header, [&](unsigned t, Rows& r) { load(t, r.a, r.b); },
+        [&](unsigned t, unsigned e, Rows& r, auto&& mid) { finish(t, e, r.a, r.b, mid); });
   }
 }
 
@@ -838,46 +883,38 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void linear_bwd_kernel(
     float* __restrict__ da, float* __restrict__ db, EwGeom g, unsigned* header,
     mg_slot_t* agg_data, mg_slot_t* incl_data) {
   constexpr bool NT = PH != EW_REDUCE;
-  // Uniform tickets: without them this kernel spills 38 registers at the cap.
-  ew_chunks<PH, true>(g, header, [&](unsigned ticket, unsigned long long epoch) {
-    EwThread th = ew_thread_at<VEC, true, true>(g, ticket, epoch);
+  ew_chunks<PH>(g, header, [&](unsigned ticket, unsigned long long epoch) {
+    EwThread th = ew_thread_at<VEC, true>(g, ticket, epoch);
     const int64_t t0 = (int64_t)th.c * (WAVES * TSUB) + th.w * TSUB;
     const int64_t T = g.T, D = g.D;
 
     // bp[s] = Bc_{t0+s-1} (zero before the sequence start).
     float av[TSUB][VEC], bp[TSUB][VEC], xa[TSUB][VEC], xb[TSUB][VEC];
     float Ap[VEC];
+    EwRows rows(th, t0, T, D);
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
-      const int64_t t = t0 + s;
-      if (th.col_ok && t < T) {
-        const int64_t off = (th.bb * T + t) * D + th.col;
-        load_vec<VEC, NT>(av[s], a + off);
-        if constexpr (PH != EW_REDUCE) {
-          if (t > 0) {
-            load_vec<VEC>(bp[s], Bc + off - D);
-          } else {
+      const int64_t off = rows.next();
+      load_vec<VEC, NT>(av[s], a + off + th.cl);
+      if constexpr (PH != EW_REDUCE)
+        load_vec<VEC>(bp[s], Bc + (t0 + s > 0 ? off - D : off) + th.cl);
+      load_vec<VEC, NT>(xa[s], gA + off + th.cl);
+      load_vec<VEC, NT>(xb[s], gB + off + th.cl);
+    }
+    load_vec<VEC>(Ap, A + th.row(t0 > 0 ? t0 - 1 : 0, T) * D + th.cl);
 #pragma unroll
-            for (int v = 0; v < VEC; ++v) bp[s][v] = 0.f;
-          }
-        }
-        load_vec<VEC, NT>(xa[s], gA + off);
-        load_vec<VEC, NT>(xb[s], gB + off);
-      } else {
+    for (int s = 0; s < TSUB; ++s) {
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) {
+      for (int v = 0; v < VEC; ++v) {
+        if (t0 + s >= T) {
           av[s][v] = 1.f;
-          bp[s][v] = 0.f;
-          xa[s][v] = 0.f;
-          xb[s][v] = 0.f;
+          xa[s][v] = xb[s][v] = 0.f;
+        }
+        if (s == 0 && t0 == 0) {
+          bp[0][v] = 0.f;
+          Ap[v] = 1.f;
         }
       }
-    }
-    if (th.col_ok && t0 > 0 && t0 <= T) {
-      load_vec<VEC>(Ap, A + (th.bb * T + t0 - 1) * D + th.col);
-    } else {
-#pragma unroll
-      for (int v = 0; v < VEC; ++v) Ap[v] = 1.f;
     }
 
     Aff<2> loc[VEC], seed[VEC], carry[VEC];
@@ -942,37 +979,34 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void linear_bwd_bf16_kernel(
     mg_slot_t* incl_data) {
   static_assert(TSUB == LIN_STATE, "one recorded state per wave");
   constexpr bool NT = PH != EW_REDUCE;
-  ew_chunks<PH, true>(g, header, [&](unsigned ticket, unsigned long long epoch) {
-    const EwThread th = ew_thread_at<VEC, true, true>(g, ticket, epoch);
+  ew_chunks<PH>(g, header, [&](unsigned ticket, unsigned long long epoch) {
+    const EwThread th = ew_thread_at<VEC, true>(g, ticket, epoch);
     const int64_t t0 = (int64_t)th.c * (WAVES * TSUB) + th.w * TSUB;
     const int64_t T = g.T, D = g.D;
 
     Raw<mg_bf16, VEC> av[TSUB], bv[TSUB], ga[TSUB], gb[TSUB];
+    EwRows rows(th, t0, T, D);
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
-      const int64_t t = t0 + s;
-      if (th.col_ok && t < T) {
-        const int64_t off = (th.bb * T + t) * D + th.col;
-        load_raw<VEC, NT>(av[s], a + off);
-        if constexpr (PH != EW_REDUCE) load_raw<VEC>(bv[s], b + off);
-        load_raw<VEC, NT>(ga[s], gA + off);
-        load_raw<VEC, NT>(gb[s], gB + off);
-      } else {
+      const int64_t off = rows.next();
+      load_raw<VEC, NT>(av[s], a + off + th.cl);
+      if constexpr (PH != EW_REDUCE) load_raw<VEC>(bv[s], b + off + th.cl);
+      load_raw<VEC, NT>(ga[s], gA + off + th.cl);
+      load_raw<VEC, NT>(gb[s], gB + off + th.cl);
+    }
+    float Ap[VEC], Bp[VEC];
+    const int64_t nsub = (T + TSUB - 1) / TSUB;
+    const float* st =
+        state + (th.bb * nsub + (t0 < T ? t0 / TSUB : nsub - 1)) * 2 * D;
+    load_vec<VEC>(Ap, st + th.cl);
+    load_vec<VEC>(Bp, st + D + th.cl);
+#pragma unroll
+    for (int s = 0; s < TSUB; ++s) {
+      if (t0 + s >= T) {
         av[s].fill(1.f);
-        bv[s].fill(0.f);
         ga[s].fill(0.f);
         gb[s].fill(0.f);
       }
-    }
-    float Ap[VEC], Bp[VEC];
-    if (PH != EW_REDUCE && th.col_ok && t0 < T) {
-      const int64_t nsub = (T + TSUB - 1) / TSUB;
-      const float* st = state + ((th.bb * nsub + t0 / TSUB) * 2) * D + th.col;
-      load_vec<VEC>(Ap, st);
-      load_vec<VEC>(Bp, st + D);
-    } else {
-#pragma unroll
-      for (int v = 0; v < VEC; ++v) Ap[v] = Bp[v] = 0.f;
     }
 
     Aff<2> loc[VEC], seed[VEC], carry[VEC];
@@ -1070,28 +1104,21 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void log_fwd_kernel(
     // Every raw load first, then the exponentials: with each step's exponentials
     // next to its loads the compiler waited for them step by step.
     float ra[TSUB][VEC], rb[TSUB][VEC];
+    EwRows rows(th, t0, T, D);
+    const int64_t to_lv = (int64_t)(th.bb + 1) * D;  // lv has a row more per batch row
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
-      const int64_t t = t0 + s;
-      if (th.col_ok && t < T) {
-        load_vec<VEC, NT>(ra[s], lc + (th.bb * T + t) * D + th.col);
-        load_vec<VEC, NT>(rb[s], lv + (th.bb * (T + 1) + t + 1) * D + th.col);
-      } else {
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) {
-          ra[s][v] = 0.f;  // unused: the step is past the end
-          rb[s][v] = 0.f;
-        }
-      }
+      const int64_t off = rows.next();
+      load_vec<VEC, NT>(ra[s], lc + off + th.cl);
+      load_vec<VEC, NT>(rb[s], lv + off + to_lv + th.cl);
     }
     Xf av[TSUB][VEC], bv[TSUB][VEC];
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
-      const bool ok = th.col_ok && t0 + s < T;
 #pragma unroll
       for (int v = 0; v < VEC; ++v) {
-        av[s][v] = ok ? xf_exp(ra[s][v]) : Xf{1.f, 0.f};
-        bv[s][v] = ok ? xf_exp(rb[s][v]) : xf_zero();
+        av[s][v] = xf_exp(ra[s][v]);
+        bv[s][v] = xf_exp(rb[s][v]);
       }
     }
 
@@ -1161,29 +1188,26 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void log_bwd_kernel(
 
     // a as Xf; lv and gh raw until needed.
     float ra[TSUB][VEC], lvr[TSUB][VEC], gr[TSUB][VEC];
+    EwRows rows(th, t0, T, D);
+    const int64_t to_lv = (int64_t)(th.bb + 1) * D;  // lv has a row more per batch row
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
-      const int64_t t = t0 + s;
-      if (th.col_ok && t < T) {
-        load_vec<VEC, NT>(ra[s], lc + (th.bb * T + t) * D + th.col);
-        if constexpr (PH != EW_REDUCE) load_vec<VEC>(lvr[s], lv + (th.bb * (T + 1) + t + 1) * D + th.col);
-        load_vec<VEC, NT>(gr[s], gh + (th.bb * T + t) * D + th.col);
-      } else {
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) {
-          ra[s][v] = 0.f;  // unused: the step is past the end
-          lvr[s][v] = -INFINITY;
-          gr[s][v] = 0.f;
-        }
-      }
+      const int64_t off = rows.next();
+      load_vec<VEC, NT>(ra[s], lc + off + th.cl);
+      if constexpr (PH != EW_REDUCE) load_vec<VEC>(lvr[s], lv + off + to_lv + th.cl);
+      load_vec<VEC, NT>(gr[s], gh + off + th.cl);
     }
     // The exponentials after every load is issued (as in the forward).
     Xf av[TSUB][VEC];
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
-      const bool ok = th.col_ok && t0 + s < T;
+      const bool ok = t0 + s < T;
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) av[s][v] = ok ? xf_exp(ra[s][v]) : Xf{1.f, 0.f};
+      for (int v = 0; v < VEC; ++v) {
+        const Xf e = xf_exp(ra[s][v]);
+        av[s][v] = ok ? e : Xf{1.f, 0.f};
+        if (!ok) gr[s][v] = 0.f;
+      }
     }
     // An fp32 value as Xf without normalising: only an exact zero needs exponent -inf.
     auto raw = [](float x) { return Xf{x, x == 0.f ? -INFINITY : 0.f}; };
@@ -1354,38 +1378,40 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void gate_fwd_kernel(
     EwGeom g, unsigned* header, mg_slot_t* agg_data, mg_slot_t* incl_data) {
   constexpr bool NT = PH != EW_REDUCE;
   constexpr bool HALF = !std::is_same_v<E, float>;
+  constexpr bool IN3 = gate_inputs<G>() == 3;
   static_assert(!HALF || TSUB % GATE_STATE == 0, "recorded states at whole sub-chunks");
-  ew_chunks<PH>(g, header, [&](unsigned ticket, unsigned long long epoch) {
-    EwThread th = ew_thread_at<VEC, false>(g, ticket, epoch);
+  const int64_t T = g.T, D = g.D;
+  struct Rows {
+    Raw<E, VEC> x0[TSUB], x1[TSUB], x2[IN3 ? TSUB : 1];
+  };
+  auto load = [&](unsigned ticket, Rows& r) {
+    const EwThread th = ew_thread_at<VEC, false>(g, ticket, 0u);
     const int64_t t0 = (int64_t)th.c * (WAVES * TSUB) + th.w * TSUB;
-    const int64_t T = g.T, D = g.D;
+    EwRows rows(th, t0, T, g.ld);
+#pragma unroll
+    for (int s = 0; s < TSUB; ++s) {
+      const int64_t off = rows.next();
+      load_raw<VEC, NT>(r.x0[s], p0 + off + th.cl);
+      load_raw<VEC, NT>(r.x1[s], p1 + off + th.cl);
+      if constexpr (IN3) load_raw<VEC, NT>(r.x2[s], p2 + off + th.cl);
+    }
+  };
+  auto finish = [&](unsigned ticket, unsigned long long epoch, Rows& r, auto&& mid) {
+    const EwThread th = ew_thread_at<VEC, false>(g, ticket, epoch);
+    const int64_t t0 = (int64_t)th.c * (WAVES * TSUB) + th.w * TSUB;
     float nlam[VEC], dts[TSUB];  // -lam log2(e) per column, dt per step
     if constexpr (DEC) {
       decay_rates<VEC>(nlam, dec.lam, th.col, D);
       decay_gaps<TSUB>(dts, dec.dt, th.bb * T + t0, T - t0, th.lane);
     }
-
     float av[TSUB][VEC], bv[TSUB][VEC];
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
-      const int64_t t = t0 + s;
-      if (th.col_ok && t < T) {
-        const int64_t off = (th.bb * T + t) * g.ld + th.col;
-        float x0[VEC], x1[VEC], x2[VEC];
-        load_vec<VEC, NT>(x0, p0 + off);
-        load_vec<VEC, NT>(x1, p1 + off);
-        if constexpr (gate_inputs<G>() == 3) load_vec<VEC, NT>(x2, p2 + off);
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) {
-          gate_coeffs<G>(x0[v], x1[v], gate_inputs<G>() == 3 ? x2[v] : 0.f, av[s][v], bv[s][v]);
-          if constexpr (DEC) av[s][v] *= __builtin_amdgcn_exp2f(nlam[v] * dts[s]);
-        }
-      } else {
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) {
-          av[s][v] = 1.f;
-          bv[s][v] = 0.f;
-        }
+      for (int v = 0; v < VEC; ++v) {
+        gate_coeffs<G>(r.x0[s].get(v), r.x1[s].get(v), IN3 ? r.x2[IN3 ? s : 0].get(v) : 0.f,
+                       av[s][v], bv[s][v]);
+        if constexpr (DEC) av[s][v] *= __builtin_amdgcn_exp2f(nlam[v] * dts[s]);
       }
     }
     Aff<1> loc[VEC], seed[VEC], carry[VEC];
@@ -1405,6 +1431,7 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void gate_fwd_kernel(
 #pragma unroll
       for (int v = 0; v < VEC; ++v) seed[v].l[0] = G == GATE_MINGRU ? expf(x[v]) : x[v];
     }
+    mid();
     ew_carry<Aff<1>, VEC, WAVES, false, PH>(loc, seed, g, th.lg, th.c, header, th.epoch, agg_data,
                                             incl_data, carry);
     if constexpr (PH == EW_REDUCE) return;
@@ -1424,7 +1451,16 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void gate_fwd_kernel(
       const int64_t t = t0 + s;
       if (th.col_ok && t < T) store_vec<VEC>(h + (th.bb * T + t) * D + th.col, L);
     }
-  });
+  };
+  if constexpr (HALF && PH == EW_LOOKBACK) {
+    ew_persistent2<Rows>(g, header, load, finish);
+  } else {
+    ew_chunks<PH>(g, header, [&](unsigned ticket, unsigned long long epoch) {
+      Rows r;
+      load(ticket, r);
+      finish(ticket, epoch, r, [] {});
+    });
+  }
 }
 
 // Backward: x_t = dL/dh_t in total (reverse scan of g_t with the a's), then
@@ -1442,14 +1478,31 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void gate_bwd_kernel(
     mg_slot_t* incl_data) {
   // dL/dlam partials of the workgroup's waves (DEC with dlam).
   __shared__ float s_dlam[DEC ? WAVES : 1][DEC ? MG_WAVE * VEC : 1];
-  ew_chunks<PH>(g, header, [&](unsigned ticket, unsigned long long epoch) {
-    EwThread th = ew_thread_at<VEC, true>(g, ticket, epoch);
+  constexpr bool MIN = G == GATE_MINGRU;
+  constexpr bool NT = PH != EW_REDUCE;
+  constexpr bool HALF = !std::is_same_v<E, float>;
+  static_assert(!HALF || TSUB == GATE_STATE, "one recorded state per wave");
+  const int64_t T = g.T, D = g.D;
+  // Rows: p0, the upstream gradient, z (signed gates) and hpre.
+  struct Rows {
+    Raw<E, VEC> x0[TSUB], gr[TSUB], x1[MIN ? 1 : TSUB], hp[TSUB];
+  };
+  auto load = [&](unsigned ticket, Rows& r) {
+    const EwThread th = ew_thread_at<VEC, true>(g, ticket, 0u);
     const int64_t t0 = (int64_t)th.c * (WAVES * TSUB) + th.w * TSUB;
-    const int64_t T = g.T, D = g.D;
-    constexpr bool MIN = G == GATE_MINGRU;
-    constexpr bool NT = PH != EW_REDUCE;
-    constexpr bool HALF = !std::is_same_v<E, float>;
-    static_assert(!HALF || TSUB == GATE_STATE, "one recorded state per wave");
+    EwRows rows(th, t0, T, g.ld), grows(th, t0, T, D);
+#pragma unroll
+    for (int s = 0; s < TSUB; ++s) {
+      const int64_t off = rows.next();
+      load_raw<VEC, NT>(r.x0[s], p0 + off + th.cl);
+      load_raw<VEC, NT>(r.gr[s], gh + grows.next() + th.cl);
+      if constexpr (!MIN) load_raw<VEC, NT>(r.x1[s], p1 + off + th.cl);
+      if constexpr (PH != EW_REDUCE) load_raw<VEC>(r.hp[s], (MIN ? p1 : p2) + off + th.cl);
+    }
+  };
+  auto finish = [&](unsigned ticket, unsigned long long epoch, Rows& r, auto&& mid) {
+    const EwThread th = ew_thread_at<VEC, true>(g, ticket, epoch);
+    const int64_t t0 = (int64_t)th.c * (WAVES * TSUB) + th.w * TSUB;
     // Decay: -lam log2(e) per column and dt per step (one value per wave and step).
     float nlam[VEC], dts[TSUB];
     if constexpr (DEC) {
@@ -1468,37 +1521,23 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void gate_bwd_kernel(
     float ua[TSUB][VEC], ub[TSUB][VEC], hv[TSUB][VEC], x[TSUB][VEC];
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
-      const int64_t t = t0 + s;
-      if (th.col_ok && t < T) {
-        const int64_t off = (th.bb * T + t) * g.ld + th.col;
-        float x0[VEC];
-        load_vec<VEC, NT>(x0, p0 + off);
-        load_vec<VEC, NT>(x[s], gh + (th.bb * T + t) * D + th.col);
+      // Steps past the end: no gradient, and a = 0 closes the adjoint chain.  (A step's
+      // values are formed before the end picks, without a branch.)
+      const bool ok = t0 + s < T;
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        const float p = r.x0[s].get(v);
+        float va, vb;
         if constexpr (MIN) {
-          if constexpr (PH != EW_REDUCE) load_vec<VEC>(hv[s], p1 + off);
-#pragma unroll
-          for (int v = 0; v < VEC; ++v) {
-            ua[s][v] = mg_sigmoid(-x0[v]);  // a
-            ub[s][v] = mg_sigmoid(x0[v]);   // z
-          }
+          mg_sigmoid_pair(p, vb, va);  // z and a
         } else {
-          float x1[VEC];
-          load_vec<VEC, NT>(x1, p1 + off);
-          if constexpr (PH != EW_REDUCE) load_vec<VEC>(hv[s], p2 + off);
-#pragma unroll
-          for (int v = 0; v < VEC; ++v) {
-            ua[s][v] = mg_sigmoid(x1[v]);  // sigmoid(z)
-            ub[s][v] = mg_tanh(x0[v]);     // tanh(s)
-          }
+          va = mg_sigmoid(r.x1[s].get(v));  // sigmoid(z)
+          vb = mg_tanh(p);                  // tanh(s)
         }
-      } else {
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) {
-          ua[s][v] = 0.f;  // a = 0 closes the adjoint chain past T
-          ub[s][v] = 0.f;
-          hv[s][v] = 0.f;
-          x[s][v] = 0.f;
-        }
+        ua[s][v] = ok ? va : 0.f;
+        ub[s][v] = ok ? vb : 0.f;
+        x[s][v] = ok ? r.gr[s].get(v) : 0.f;
+        if constexpr (PH != EW_REDUCE) hv[s][v] = ok ? r.hp[s].get(v) : 0.f;
       }
     }
     auto coef_a0 = [&](int s, int v) {  // the coefficient before decay
@@ -1509,22 +1548,15 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void gate_bwd_kernel(
     auto coef_a = [&](int s, int v) { return DEC ? coef_a0(s, v) * gam(s, v) : coef_a0(s, v); };
     const bool first_sub = (t0 == 0);
     float hprev[VEC];
-    if (HALF ? th.col_ok && t0 < T : th.col_ok && t0 <= T) {
-      if constexpr (HALF) {
-        const int64_t nsub = (T + TSUB - 1) / TSUB;
-        load_vec<VEC>(hprev, h + (th.bb * nsub + t0 / TSUB) * D + th.col);
-      } else if (first_sub) {
-        load_vec<VEC>(hprev, h0 + th.bb * D + th.col);
-        if constexpr (MIN) {
-#pragma unroll
-          for (int v = 0; v < VEC; ++v) hprev[v] = expf(hprev[v]);
-        }
-      } else {
-        load_vec<VEC>(hprev, h + (th.bb * T + t0 - 1) * D + th.col);
-      }
+    if constexpr (HALF) {
+      const int64_t nsub = (T + TSUB - 1) / TSUB;
+      load_vec<VEC>(hprev, h + (th.bb * nsub + (t0 < T ? t0 / TSUB : nsub - 1)) * D + th.cl);
     } else {
+      load_vec<VEC>(hprev, (first_sub ? h0 + th.bb * D : h + th.row(t0 - 1, T) * D) + th.cl);
+      if (MIN && first_sub) {
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) hprev[v] = 0.f;
+        for (int v = 0; v < VEC; ++v) hprev[v] = expf(hprev[v]);
+      }
     }
 
     Aff<1> loc[VEC], seed[VEC], carry[VEC];
@@ -1539,6 +1571,7 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void gate_bwd_kernel(
       }
       seed[v] = aff_identity<1>();
     }
+    mid();
     ew_carry<Aff<1>, VEC, WAVES, true, PH>(loc, seed, g, th.lg, th.c, header, th.epoch, agg_data,
                                            incl_data, carry);
     if constexpr (PH == EW_REDUCE) return;
@@ -1578,7 +1611,7 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void gate_bwd_kernel(
         if constexpr (MIN) {
           // a = sigmoid(-k): da/dk = -a z;  b = z g(hpre): db/dk = z a g, db/dhpre = z g'.
           const float hp = hv[s][v], am = ua[s][v], zk = ub[s][v];
-          const float gv = hp >= 0.f ? hp + 0.5f : mg_sigmoid(hp);
+          const float gv = mg_g(hp);
           const float gp = hp >= 0.f ? 1.f : gv * (1.f - gv);
           a = am;
           b = zk * gv;
@@ -1638,7 +1671,16 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void gate_bwd_kernel(
         __syncthreads();  // s_dlam is free for the workgroup's next chunk
       }
     }
-  });
+  };
+  if constexpr (HALF && PH == EW_LOOKBACK) {
+    ew_persistent2<Rows>(g, header, load, finish);
+  } else {
+    ew_chunks<PH>(g, header, [&](unsigned ticket, unsigned long long epoch) {
+      Rows r;
+      load(ticket, r);
+      finish(ticket, epoch, r, [] {});
+    });
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1711,7 +1753,8 @@ int ew_launch(Kernel k, const EwPlan& p, void* ws, hipStream_t stream, bool pers
   mg_slot_t* incl = (mg_slot_t*)((char*)ws + p.incl_off);
   const unsigned chunks = (unsigned)p.g.n_lg * (unsigned)p.g.n_chunks;
   const unsigned grid =
-      persistent ? std::min(chunks, mg_resident((const void*)k, MG_WAVE * p.waves)) : chunks;
+      persistent ? std::min(chunks, mg_resident((const void*)k, MG_WAVE * p.waves, EW_MAX_PER_CU))
+                 : chunks;
   hipLaunchKernelGGL(k, dim3(grid), dim3(MG_WAVE * p.waves), 0, stream, args..., p.g, header,
                      agg, incl);
   return hipGetLastError() == hipSuccess ? MG_OK : MG_ERR_LAUNCH;

@@ -18,13 +18,27 @@ __device__ __forceinline__ float mg_sigmoid(float x) {
   return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504088896341f * x));
 }
 __device__ __forceinline__ float mg_tanh(float x) { return fmaf(2.f, mg_sigmoid(2.f * x), -1.f); }
-__device__ __forceinline__ float mg_g(float x) { return x >= 0.f ? x + 0.5f : mg_sigmoid(x); }
+// sigmoid(x) and sigmoid(-x) from one exponential: with e = e^-|x| in (0, 1],
+// sigmoid(|x|) = 1 / (1 + e) and sigmoid(-|x|) = e / (1 + e), so neither overflows and
+// both keep the relative error of mg_sigmoid (an exp2 and a reciprocal, one rounding more).
+__device__ __forceinline__ void mg_sigmoid_pair(float x, float& pos, float& neg) {
+  const float e = __builtin_amdgcn_exp2f(-1.44269504088896341f * fabsf(x));
+  const float big = __builtin_amdgcn_rcpf(1.f + e), small = e * big;
+  pos = x >= 0.f ? big : small;
+  neg = x >= 0.f ? small : big;
+}
+// The sigmoid is formed before the sign picks: as an arm of the conditional it became a
+// branch per element, which also kept a chunk's loads from being issued together.
+__device__ __forceinline__ float mg_g(float x) {
+  const float sg = mg_sigmoid(x);
+  return x >= 0.f ? x + 0.5f : sg;
+}
 
 template <int G>
 __device__ __forceinline__ void gate_coeffs(float p0, float p1, float p2, float& a, float& b) {
   if constexpr (G == GATE_MINGRU) {
-    a = mg_sigmoid(-p0);
-    b = mg_sigmoid(p0) * mg_g(p1);
+    mg_sigmoid_pair(p0, b, a);
+    b *= mg_g(p1);
   } else {
     const float sg = mg_sigmoid(p1), th = mg_tanh(p0);
     a = G == GATE_SIGNED_COUPLED ? (1.f - sg) * th : th;
