@@ -333,15 +333,26 @@ int mg_log_scan_bf16_fwd(const void* lc, const void* lv, void* h, float* hstate,
 int mg_log_scan_bf16_bwd(const void* lc, const void* lv, const float* hstate, const void* gh,
                          void* dlc, void* dlv, int64_t B, int64_t T, int64_t D, void* ws,
                          size_t ws_bytes, mg_stream_t stream);
-/* The fused gate scans: kind 0 SignedMinGRU (p0, p1, p2 = s, z, hpre), 1 coupled, 2
+/* The fused gate scans over pre-activations with a row stride: kind 0 SignedMinGRU (p0, p1, p2 = s, z, hpre), 1 coupled, 2
  * MinGRU (p0, p1 = k, hpre; p2, d2 unused; h0 = log h0).  p* and d* rows lie `ld` (>= D)
- * elements apart; h0 (B,D) is bf16 (h0_half = 1) or fp32; dt (B,T) and lam (D) are given
+ * elements apart (slices of one projection's rows, say); h0 (B,D) is bf16 (h0_half = 1) or
+ * fp32, or NULL: every initial state is then h0_const; dt (B,T) and lam (D) are given
  * together (time decay) or both NULL; dlam and ddt as mg_signed_gate_scan_decay_bwd,
- * each may be NULL; dh0 is fp32. */
+ * each may be NULL; dh0 is fp32 and may be NULL.  mg_gate_scan_rows_*: the same on fp32
+ * tensors, the backward restarting from the forward's h. */
+int mg_gate_scan_rows_fwd(int kind, const float* p0, const float* p1, const float* p2, int64_t ld,
+                          const float* h0, float h0_const, const float* dt, const float* lam,
+                          float* h, int64_t B, int64_t T, int64_t D, void* ws, size_t ws_bytes,
+                          mg_stream_t stream);
+int mg_gate_scan_rows_bwd(int kind, const float* p0, const float* p1, const float* p2, int64_t ld,
+                          const float* h0, float h0_const, const float* dt, const float* lam,
+                          const float* h, const float* gh, float* d0, float* d1, float* d2,
+                          float* dh0, float* dlam, float* ddt, int64_t B, int64_t T, int64_t D,
+                          void* ws, size_t ws_bytes, mg_stream_t stream);
 size_t mg_gate_scan_bf16_state_bytes(int64_t B, int64_t T, int64_t D);
 int mg_gate_scan_bf16_fwd(int kind, const void* p0, const void* p1, const void* p2, int64_t ld,
-                          const void* h0, int h0_half, const float* dt, const float* lam, void* h,
-                          float* state, int64_t B, int64_t T, int64_t D, void* ws,
+                          const void* h0, int h0_half, float h0_const, const float* dt,
+                          const float* lam, void* h, float* state, int64_t B, int64_t T, int64_t D, void* ws,
                           size_t ws_bytes, mg_stream_t stream);
 int mg_gate_scan_bf16_bwd(int kind, const void* p0, const void* p1, const void* p2, int64_t ld,
                           const float* dt, const float* lam, const float* state, const void* gh,

@@ -27,6 +27,7 @@ MG_STATUS = {
 _P = ctypes.c_void_p
 _I64 = ctypes.c_int64
 _I32 = ctypes.c_int
+_F32 = ctypes.c_float
 _SZ = ctypes.c_size_t
 
 _SIGNATURES = {
@@ -55,7 +56,14 @@ _SIGNATURES = {
     "mg_log_scan_bf16_bwd": (_I32, [_P] * 6 + [_I64, _I64, _I64, _P, _SZ, _P]),
     "mg_gate_scan_bf16_state_bytes": (_SZ, [_I64, _I64, _I64]),
     "mg_gate_scan_bf16_fwd": (
-        _I32, [_I32] + [_P] * 3 + [_I64, _P, _I32] + [_P] * 4 + [_I64, _I64, _I64, _P, _SZ, _P],
+        _I32,
+        [_I32] + [_P] * 3 + [_I64, _P, _I32, _F32] + [_P] * 4 + [_I64, _I64, _I64, _P, _SZ, _P],
+    ),
+    "mg_gate_scan_rows_fwd": (
+        _I32, [_I32] + [_P] * 3 + [_I64, _P, _F32] + [_P] * 3 + [_I64, _I64, _I64, _P, _SZ, _P],
+    ),
+    "mg_gate_scan_rows_bwd": (
+        _I32, [_I32] + [_P] * 3 + [_I64, _P, _F32] + [_P] * 10 + [_I64, _I64, _I64, _P, _SZ, _P],
     ),
     "mg_gate_scan_bf16_bwd": (
         _I32, [_I32] + [_P] * 3 + [_I64] + [_P] * 10 + [_I64, _I64, _I64, _P, _SZ, _P],

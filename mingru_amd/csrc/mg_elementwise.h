@@ -330,6 +330,7 @@ struct EwGeom {
   int64_t T, D;
   int n_tiles, n_lg, n_chunks;
   int64_t ld;   // gate scans: elements between rows of the pre-activations and their gradients
+  float h0_const;  // gate scans: every initial state where no h0 tensor is given
   int h0_half;  // gate scans of bf16 elements: the initial state is bf16 too (fp32 otherwise)
 };
 
@@ -1357,13 +1358,19 @@ __device__ __forceinline__ void decay_gaps(float (&dts)[TSUB], const float* dt, 
     dts[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), s));
 }
 
-// The initial state of the thread's columns: E's type, or fp32 with bf16 elements.
+// The initial state of the thread's columns: E's type, or fp32 with bf16 elements, or
+// g.h0_const where there is no tensor.
 template <typename E, int VEC>
-__device__ __forceinline__ void load_h0(float (&x)[VEC], const void* h0, int64_t off, int half) {
-  if (!std::is_same_v<E, float> && half)
+__device__ __forceinline__ void load_h0(float (&x)[VEC], const void* h0, int64_t off,
+                                        const EwGeom& g) {
+  if (h0 == nullptr) {
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) x[v] = g.h0_const;
+  } else if (!std::is_same_v<E, float> && g.h0_half) {
     load_vec<VEC>(x, (const E*)h0 + off);
-  else
+  } else {
     load_vec<VEC>(x, (const float*)h0 + off);
+  }
 }
 
 // bf16 elements (E): h is rounded to bf16, so the forward records the fp32 state before
@@ -1427,7 +1434,7 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void gate_fwd_kernel(
     }
     if (th.c == 0 && th.w == 0 && th.col_ok) {
       float x[VEC];
-      load_h0<E, VEC>(x, h0, th.bb * D + th.col, g.h0_half);
+      load_h0<E, VEC>(x, h0, th.bb * D + th.col, g);
 #pragma unroll
       for (int v = 0; v < VEC; ++v) seed[v].l[0] = G == GATE_MINGRU ? expf(x[v]) : x[v];
     }
@@ -1552,7 +1559,10 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void gate_bwd_kernel(
       const int64_t nsub = (T + TSUB - 1) / TSUB;
       load_vec<VEC>(hprev, h + (th.bb * nsub + (t0 < T ? t0 / TSUB : nsub - 1)) * D + th.cl);
     } else {
-      load_vec<VEC>(hprev, (first_sub ? h0 + th.bb * D : h + th.row(t0 - 1, T) * D) + th.cl);
+      if (first_sub)
+        load_h0<float, VEC>(hprev, h0, th.bb * D + th.cl, g);
+      else
+        load_vec<VEC>(hprev, h + th.row(t0 - 1, T) * D + th.cl);
       if (MIN && first_sub) {
 #pragma unroll
         for (int v = 0; v < VEC; ++v) hprev[v] = expf(hprev[v]);
@@ -1586,7 +1596,7 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void gate_bwd_kernel(
         y[v] = coef_a(s, v) * x[s][v];
       }
     }
-    if (first_sub && th.col_ok) {
+    if (first_sub && th.col_ok && dh0 != nullptr) {
       // dL/dh0 = a_1 x_1; the MinGRU input is log h0: times h0.
       if constexpr (MIN) {
 #pragma unroll
@@ -1700,6 +1710,7 @@ EwPlan ew_plan(int64_t B, int64_t T, int64_t D, int vec, int tsub, int waves, in
   p.g.D = D;
   p.g.ld = D;
   p.g.h0_half = 0;
+  p.g.h0_const = 0.f;
   const int tile = MG_WAVE * vec;
   p.g.n_tiles = (int)((D + tile - 1) / tile);
   p.g.n_lg = (int)(B * p.g.n_tiles);
@@ -1840,6 +1851,7 @@ struct GateIn {
   const void *p0, *p1, *p2, *h0;
   int64_t ld;
   int h0_half;
+  float h0_const = 0.f;  // the initial state where h0 is null
 };
 
 template <typename E, int G, bool DEC>
@@ -1856,6 +1868,7 @@ int gate_fwd_launch(const GateIn& in, void* h, float* hstate, GateDecay dec, int
     if (ws_bytes < p.total) return MG_ERR_WORKSPACE;
     p.g.ld = in.ld;
     p.g.h0_half = in.h0_half;
+    p.g.h0_const = in.h0_const;
     return ew_run(ew_two_launch(p, B, T, D, gate_inputs<G>(), sizeof(E)),
                   gate_fwd_kernel<E, V, TS, EW_WAVES_FWD, G, DEC>,
                   gate_fwd_kernel<E, V, TS, EW_WAVES_FWD, G, DEC, EW_REDUCE>,
@@ -1879,6 +1892,7 @@ int gate_bwd_launch(const GateIn& in, const float* h, const void* gh, void* d0, 
     EwPlan p = ew_plan(B, T, D, V, GATE_TSUB_BWD, GATE_WAVES_BWD, 1);
     if (ws_bytes < p.total) return MG_ERR_WORKSPACE;
     p.g.ld = in.ld;
+    p.g.h0_const = in.h0_const;
     return ew_run(ew_two_launch(p, B, T, D, gate_inputs<G>() + 1, sizeof(E)),
                   gate_bwd_kernel<E, V, GATE_TSUB_BWD, GATE_WAVES_BWD, G, DEC>,
                   gate_bwd_kernel<E, V, GATE_TSUB_BWD, GATE_WAVES_BWD, G, DEC, EW_REDUCE>,

@@ -242,6 +242,30 @@ int mg_mingru_gate_scan_decay_bwd(const float* k, const float* hpre, const float
                              ws_bytes, stream);
 }
 
+int mg_gate_scan_rows_fwd(int kind, const float* p0, const float* p1, const float* p2, int64_t ld,
+                          const float* h0, float h0_const, const float* dt, const float* lam,
+                          float* h, int64_t B, int64_t T, int64_t D, void* ws, size_t ws_bytes,
+                          hipStream_t stream) {
+  if (kind < GATE_SIGNED || kind > GATE_MINGRU || !p0 || !p1 || (kind != GATE_MINGRU && !p2) ||
+      !h || !ws || !geometry_ok(B, T, D) || ld < D || !dt != !lam)
+    return MG_ERR_ARG;
+  return gate_fwd_any<float>(kind, {p0, p1, p2, h0, ld, 0, h0_const}, h, nullptr,
+                             GateDecay{dt, lam, nullptr, nullptr}, B, T, D, ws, ws_bytes, stream);
+}
+
+int mg_gate_scan_rows_bwd(int kind, const float* p0, const float* p1, const float* p2, int64_t ld,
+                          const float* h0, float h0_const, const float* dt, const float* lam,
+                          const float* h, const float* gh, float* d0, float* d1, float* d2,
+                          float* dh0, float* dlam, float* ddt, int64_t B, int64_t T, int64_t D,
+                          void* ws, size_t ws_bytes, hipStream_t stream) {
+  if (kind < GATE_SIGNED || kind > GATE_MINGRU || !p0 || !p1 || (kind != GATE_MINGRU && !p2) ||
+      !h || !gh || !d0 || !d1 || (kind != GATE_MINGRU && !d2) || !ws || !geometry_ok(B, T, D) ||
+      ld < D || !dt != !lam)
+    return MG_ERR_ARG;
+  return gate_bwd_any<float>(kind, {p0, p1, p2, h0, ld, 0, h0_const}, h, gh, d0, d1, d2, dh0,
+                             GateDecay{dt, lam, dlam, ddt}, B, T, D, ws, ws_bytes, stream);
+}
+
 int64_t mg_gate_decay_dlam_rows(int64_t B, int64_t T, int64_t D) {
   if (B <= 0 || T <= 0 || D <= 0) return 0;
   return B * ((T + GATE_WAVES_BWD * GATE_TSUB_BWD - 1) / (GATE_WAVES_BWD * GATE_TSUB_BWD));

@@ -69,13 +69,13 @@ size_t mg_gate_scan_bf16_state_bytes(int64_t B, int64_t T, int64_t D) {
 }
 
 int mg_gate_scan_bf16_fwd(int kind, const void* p0, const void* p1, const void* p2, int64_t ld,
-                          const void* h0, int h0_half, const float* dt, const float* lam, void* h,
-                          float* hstate, int64_t B, int64_t T, int64_t D, void* ws,
+                          const void* h0, int h0_half, float h0_const, const float* dt,
+                          const float* lam, void* h, float* hstate, int64_t B, int64_t T, int64_t D, void* ws,
                           size_t ws_bytes, hipStream_t stream) {
   if (kind < GATE_SIGNED || kind > GATE_MINGRU || !p0 || !p1 || (kind != GATE_MINGRU && !p2) ||
-      !h0 || !h || !ws || !geometry_ok(B, T, D) || ld < D || !dt != !lam || (h0_half & ~1))
+      !h || !ws || !geometry_ok(B, T, D) || ld < D || !dt != !lam || (h0_half & ~1))
     return MG_ERR_ARG;
-  return gate_fwd_any<mg_bf16>(kind, {p0, p1, p2, h0, ld, h0_half}, h, hstate,
+  return gate_fwd_any<mg_bf16>(kind, {p0, p1, p2, h0, ld, h0_half, h0_const}, h, hstate,
                                GateDecay{dt, lam, nullptr, nullptr}, B, T, D, ws, ws_bytes,
                                stream);
 }
@@ -86,7 +86,7 @@ int mg_gate_scan_bf16_bwd(int kind, const void* p0, const void* p1, const void* 
                           int64_t B, int64_t T, int64_t D, void* ws, size_t ws_bytes,
                           hipStream_t stream) {
   if (kind < GATE_SIGNED || kind > GATE_MINGRU || !p0 || !p1 || (kind != GATE_MINGRU && !p2) ||
-      !hstate || !gh || !d0 || !d1 || (kind != GATE_MINGRU && !d2) || !dh0 || !ws ||
+      !hstate || !gh || !d0 || !d1 || (kind != GATE_MINGRU && !d2) || !ws ||
       !geometry_ok(B, T, D) || ld < D || !dt != !lam)
     return MG_ERR_ARG;
   return gate_bwd_any<mg_bf16>(kind, {p0, p1, p2, nullptr, ld, 0}, hstate, gh, d0, d1, d2, dh0,

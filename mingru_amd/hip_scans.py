@@ -38,6 +38,7 @@ __all__ = [
     "delta_gated_scan_impl",
     "signed_gate_scan_impl",
     "mingru_gate_scan_impl",
+    "gate_scan_packed_impl",
     "gate_step_impl",
     "delta_step_impl",
     "workspace_errors",
@@ -510,7 +511,7 @@ class _GateScanBf16Fn(torch.autograd.Function):
                                 dtype=torch.float32, device=q0.device)
         ws = _scan_workspace(_size("mg_signed_gate_scan_workspace_bytes", Bn, T, D), q0.device)
         _call("mg_gate_scan_bf16_fwd", kind, _ptr(q0), _ptr(q1), _ptr(q2), D, _ptr(h0c),
-              int(half), _ptr(dt32), _ptr(lam32), _ptr(h), _ptr(state), Bn, T, D, _ptr(ws),
+              int(half), 0.0, _ptr(dt32), _ptr(lam32), _ptr(h), _ptr(state), Bn, T, D, _ptr(ws),
               ws.numel(), _stream(q0))
         _check_workspace(ws, q0)
         ctx.save_for_backward(q0, q1, q2, state, dt32, lam32)
@@ -540,6 +541,114 @@ class _GateScanBf16Fn(torch.autograd.Function):
         g_dt = ddt.sum(0).to(dtd) if ddt is not None else None
         g_lam = dlam.sum(0).to(lamd) if dlam is not None else None
         return d0, d1, d2, dh0.to(d0.dtype), g_dt, g_lam, None
+
+
+class _PackedGateScan:
+    """The fused gate scans on one (B, T, n D) tensor whose rows hold the n pre-activations
+    side by side -- the output of one joined projection -- in fp32 or bf16; the backward
+    returns its whole gradient, laid out the same.  ``h0`` is None (every initial state is
+    ``h0_const``) or a (B, 1, D) tensor."""
+
+    @staticmethod
+    def forward(ctx, P, h0, dt, lam, kind, h0_const):
+        half = P.dtype == torch.bfloat16
+        P = _contig(P, P.dtype)
+        n = 2 if kind == GATE_STEP_KINDS["mingru"] else 3
+        Bn, T, N = P.shape
+        D = N // n
+        h0_half = False
+        if h0 is not None:
+            h0_half = half and h0.dtype == torch.bfloat16
+            h0 = _contig(h0, torch.bfloat16) if h0_half else _as_f32(h0)[0]
+        h = torch.empty(Bn, T, D, dtype=P.dtype, device=P.device)
+        dt32, lam32 = (None, None) if dt is None else _decay_args(dt, lam, h)
+        ws = _scan_workspace(_size("mg_signed_gate_scan_workspace_bytes", Bn, T, D), P.device)
+        base, step = P.data_ptr(), D * P.element_size()
+        pre = (base, base + step, base + 2 * step if n == 3 else 0, N)
+        end = (Bn, T, D, _ptr(ws), ws.numel(), _stream(P))
+        if half:
+            back = None
+            if any(ctx.needs_input_grad):
+                back = torch.empty(_size("mg_gate_scan_bf16_state_bytes", Bn, T, D) // 4,
+                                   dtype=torch.float32, device=P.device)
+            _call("mg_gate_scan_bf16_fwd", kind, *pre, _ptr(h0), int(h0_half), h0_const,
+                  _ptr(dt32), _ptr(lam32), _ptr(h), _ptr(back), *end)
+        else:
+            back = h
+            _call("mg_gate_scan_rows_fwd", kind, *pre, _ptr(h0), h0_const, _ptr(dt32),
+                  _ptr(lam32), _ptr(h), *end)
+        _check_workspace(ws, P)
+        ctx.save_for_backward(P, h0, back, dt32, lam32)
+        ctx.meta = (kind, h0_const, n, None if dt is None else dt.dtype,
+                    None if lam is None else lam.dtype)
+        return h
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, gh):
+        P, h0, back, dt32, lam32 = ctx.saved_tensors
+        kind, h0_const, n, dtd, lamd = ctx.meta
+        Bn, T, N = P.shape
+        D = N // n
+        gh = _contig(gh, P.dtype)
+        dP = torch.empty_like(P)
+        need = ctx.needs_input_grad
+        dh0 = torch.empty(Bn, 1, D, dtype=torch.float32, device=P.device) if need[1] else None
+        dlam = ddt = None
+        if dt32 is not None:
+            dlam, ddt = _decay_partials((Bn, T, D), need[3], need[2], P.device)
+        ws = _scan_workspace(_size("mg_signed_gate_scan_workspace_bytes", Bn, T, D), P.device)
+        step = D * P.element_size()
+
+        def slices(t):
+            base = t.data_ptr()
+            return base, base + step, base + 2 * step if n == 3 else 0
+
+        end = (_ptr(dh0), _ptr(dlam), _ptr(ddt), Bn, T, D, _ptr(ws), ws.numel(), _stream(P))
+        if P.dtype == torch.bfloat16:
+            _call("mg_gate_scan_bf16_bwd", kind, *slices(P), N, _ptr(dt32), _ptr(lam32),
+                  _ptr(back), _ptr(gh), *slices(dP), *end)
+        else:
+            _call("mg_gate_scan_rows_bwd", kind, *slices(P), N, _ptr(h0), h0_const, _ptr(dt32),
+                  _ptr(lam32), _ptr(back), _ptr(gh), *slices(dP), *end)
+        _check_workspace(ws, P)
+        return (dP, None if dh0 is None else dh0.to(P.dtype),
+                None if ddt is None else ddt.sum(0).to(dtd),
+                None if dlam is None else dlam.sum(0).to(lamd), None, None)
+
+
+class _PackedSignedGateScanFn(_PackedGateScan, torch.autograd.Function):
+    pass
+
+
+class _PackedMinGRUGateScanFn(_PackedGateScan, torch.autograd.Function):
+    pass
+
+
+def gate_scan_packed_impl(kind: str, P: torch.Tensor, h0: torch.Tensor | None,
+                          dt: torch.Tensor | None = None, lam: torch.Tensor | None = None, *,
+                          h0_const: float = 0.0):
+    """``signed_gate_scan_impl`` / ``mingru_gate_scan_impl`` on one joined projection.
+
+    ``P`` (B, T, n D) holds the pre-activations side by side in fp32 or bf16: ``s, z, hpre``
+    for ``kind`` ``"signed"`` / ``"signed_coupled"``, ``k, hpre`` for ``"mingru"``.  ``h0``
+    is (B, 1, D) (``log h0`` for ``"mingru"``), or None for ``h0_const`` everywhere.
+    Differentiable in ``P``, ``h0``, ``dt`` and ``lam``.  Declines (``ScanFallback``) what
+    the joined form does not take; the caller then runs the separate projections.
+    """
+    n = 2 if kind == "mingru" else 3
+    if kind not in GATE_STEP_KINDS or P.ndim != 3 or P.shape[2] % n or P.numel() == 0:
+        raise ScanFallback(f"joined gate scan: {kind!r} on {tuple(P.shape)}")
+    if P.dtype not in (torch.float32, torch.bfloat16):
+        raise ScanFallback(f"joined gate scan needs fp32 or bf16 (got {P.dtype})")
+    Bn, T, D = P.shape[0], P.shape[1], P.shape[2] // n
+    like = P[..., :D]
+    _same_device(P, *([] if h0 is None else [h0]))
+    if h0 is not None and tuple(h0.shape) != (Bn, 1, D):
+        raise ScanFallback(f"joined gate scan: h0 {tuple(h0.shape)}, need {(Bn, 1, D)}")
+    _check_decay("joined gate scan", like, dt, lam)
+    fn = _PackedMinGRUGateScanFn if kind == "mingru" else _PackedSignedGateScanFn
+    return _funnel("joined gate scan", fn.apply, P, h0, dt, lam, GATE_STEP_KINDS[kind], h0_const)
 
 
 def _check_decay(what: str, like: torch.Tensor, dt, lam) -> None:

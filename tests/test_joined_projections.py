@@ -1,0 +1,144 @@
+"""The joined projections: which layers they stand in for (CPU, a fake backend), and that
+the joined form equals the separate one (GPU).
+
+A no-op forward hook on one projection makes a module run its projections separately, so
+the GPU cases compare the two forms of one module.  Both compute the same sums in another
+order: fp32 results agree to about sqrt(K) 2^-24 of the largest term, bf16 ones to bf16's
+2^-8 of each output, doubled where the input's gradient sums separately rounded products.
+"""
+
+import copy
+import sys
+import types
+
+import pytest
+import torch
+from torch import nn
+
+import mingru_amd
+from mingru_amd import MinGRU, SignedMinGRU
+from mingru_amd import min_gru as mg
+
+BACKEND = "mingru_amd.hip_scans"
+
+
+def _fake(monkeypatch, calls):
+    class FakeFallback(Exception):
+        pass
+
+    def joined(kind, P, h0, dt=None, lam=None, *, h0_const=0.0):
+        calls.append(("joined", kind, tuple(P.shape), h0 is None))
+        return P[..., : P.shape[-1] // (2 if kind == "mingru" else 3)]
+
+    fake = types.ModuleType(BACKEND)
+    fake.ScanFallback = FakeFallback
+    fake.available = lambda: True
+    fake.SCAN_IMPLS = {}
+    fake.gate_scan_packed_impl = joined
+    fake.mingru_gate_scan_impl = lambda k, h, h0, *a: calls.append(("separate",)) or k
+    fake.signed_gate_scan_impl = lambda s, z, h, h0, **kw: calls.append(("separate",)) or s
+    monkeypatch.setitem(sys.modules, BACKEND, fake)
+    monkeypatch.setattr(mingru_amd, "hip_scans", fake, raising=False)
+    monkeypatch.setenv("MINGRU_SCAN", "hip")
+
+
+class _MyLinear(nn.Linear):
+    pass
+
+
+def test_plain_projections_are_joined(monkeypatch):
+    calls = []
+    _fake(monkeypatch, calls)
+    x = torch.randn(2, 5, 4)
+    m = MinGRU(4, 6)
+    out = m(x)  # the fake returns the first projection's slice
+    assert calls == [("joined", "mingru", (2, 5, 12), True)]
+    torch.testing.assert_close(out, m.linear_z(x))
+    calls.clear()
+    s = SignedMinGRU(4, 6, coupled=True, learnable_h0=True)
+    torch.testing.assert_close(s(x), s.linear_s(x))
+    assert calls == [("joined", "signed_coupled", (2, 5, 18), False)]
+
+
+@pytest.mark.parametrize("why", ["hook", "pre_hook", "subclass", "frozen", "half", "no_grad_rows",
+                                 "patched_forward", "mixed_bias"])
+def test_other_projections_stay_separate(monkeypatch, why):
+    calls = []
+    _fake(monkeypatch, calls)
+    m = MinGRU(4, 6)
+    x = torch.randn(2, 5, 4)
+    seen = []
+    if why == "hook":
+        m.linear_h.register_forward_hook(lambda *a: seen.append(1))
+    elif why == "pre_hook":
+        m.linear_h.register_forward_pre_hook(lambda *a: seen.append(1))
+    elif why == "subclass":
+        m.linear_h = _MyLinear(4, 6)
+    elif why == "frozen":
+        m.linear_h.weight.requires_grad_(False)
+    elif why == "half":
+        m, x = m.double(), x.double()
+    elif why == "patched_forward":
+        m.linear_h.forward = lambda v: seen.append(1) or nn.functional.linear(
+            v, m.linear_h.weight, m.linear_h.bias)
+    elif why == "mixed_bias":
+        m.linear_h = nn.Linear(4, 6, bias=False)
+    if why == "no_grad_rows":
+        with torch.no_grad():
+            m(x)
+    else:
+        m(x)
+    assert calls == [("separate",)]
+    if why in ("hook", "pre_hook", "patched_forward"):
+        assert seen == [1]
+
+
+def _pair(cuda, m, dtype):
+    joined = m.to(cuda, dtype)
+    separate = copy.deepcopy(joined)
+    for lin in separate.modules():
+        if isinstance(lin, nn.Linear):
+            lin.register_forward_hook(lambda *a: None)
+    return joined, separate
+
+
+MODULES = [
+    # constructor, B, T, time decay
+    (lambda: MinGRU(24, 48), 3, 200, False),
+    (lambda: MinGRU(40, 33, bias=False, learnable_h0=True), 2, 1100, False),
+    (lambda: MinGRU(16, 130, decay="learnable"), 2, 70, True),
+    (lambda: SignedMinGRU(24, 48), 1, 1, False),
+    (lambda: SignedMinGRU(64, 256, coupled=True, learnable_h0=True), 3, 777, False),
+    (lambda: SignedMinGRU(32, 520, decay="fixed"), 2, 2100, True),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", range(len(MODULES)))
+def test_joined_equals_separate(cuda, case, dtype, monkeypatch):
+    build, B, T, decay = MODULES[case]
+    print(f"[gpu] joined projections case={case} {dtype}", flush=True)
+    monkeypatch.setenv("MINGRU_SCAN", "hip")
+    torch.manual_seed(100 + case)
+    joined, separate = _pair(cuda, build(), dtype)
+    d = joined.input_size
+    x = torch.randn(B, T, d, device=cuda, dtype=dtype)
+    dt = torch.rand(B, T, device=cuda, dtype=dtype) if decay else None
+    res = []
+    calls = []
+    real = mg._join_linears
+    monkeypatch.setattr(mg, "_join_linears", lambda *a: calls.append(1) or real(*a))
+    for m in (joined, separate):
+        xi = x.clone().requires_grad_()
+        y = m(xi, delta_t=dt) if decay else m(xi)
+        gy = torch.randn(y.shape, generator=torch.Generator().manual_seed(9)).to(cuda, dtype)
+        grads = torch.autograd.grad(y, [xi, *m.parameters()], gy)
+        res.append([y.detach(), *grads])
+    torch.cuda.synchronize()
+    assert calls == [1]
+    rel = 2e-5 if dtype == torch.float32 else 2.0**-6
+    for i, (a, b) in enumerate(zip(*res)):
+        assert a.dtype == b.dtype and a.shape == b.shape
+        off = (a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-30)
+        assert off <= rel, f"output {i}: relative difference {off.item():.2e}"
