@@ -314,6 +314,20 @@ int mg_delta_gated_bwd(const void* Q, const void* K, const void* V, const void* 
                        int dk, int dv, int chunk, int dtype, void* ws, size_t ws_bytes,
                        mg_stream_t stream);
 
+/* ---- DeltaMinGRU heads from one joined projection ----------------------------------
+ * Replaces the mixer's eager head split, key normalisation, beta = 2 sigmoid(.) and
+ * layout change (src/mingru/min_gru.py:3040-3100).  P (B,T,N), N = H (dk + nh (dk + dv)
+ * + nh), rows q (H,dk) | k (nh,H,dk) | v (nh,H,dv) | beta (nh,H), in dtype (0 fp32,
+ * 1 bf16) -> Q (B,H,T,dk), K (B,H,T,nh,dk) of unit norm, V (B,H,T,nh,dv), beta (B,H,T,nh)
+ * and, if not NULL, nrm (B,H,T,nh) fp32: the keys' norms (at least 1e-12, negated where
+ * that bound was taken), which the backward needs.  dk, dv <= 64. */
+int mg_delta_heads_fwd(const void* P, void* Q, void* K, void* V, void* beta, float* nrm, int64_t B,
+                       int64_t T, int H, int nh, int dk, int dv, int dtype, mg_stream_t stream);
+/* K, beta, nrm = the forward's; dQ, dK, dV, dbeta in the kernel layouts -> dP (B,T,N). */
+int mg_delta_heads_bwd(const void* K, const void* beta, const float* nrm, const void* dQ,
+                       const void* dK, const void* dV, const void* dbeta, void* dP, int64_t B,
+                       int64_t T, int H, int nh, int dk, int dv, int dtype, mg_stream_t stream);
+
 /* ---- elementwise scans on bf16 tensors --------------------------------------------
  * The scans above with bf16 tensors (void*), computed in fp32.  No reference
  * kernels: the reference casts to fp32 around its fp32 kernels

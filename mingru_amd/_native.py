@@ -97,6 +97,8 @@ _SIGNATURES = {
     "mg_angle_scan_tables_bwd": (
         _I32, [_P] * 15 + [_I64, _I64, _I64] + [_I32] * 4 + [_P, _SZ, _P],
     ),
+    "mg_delta_heads_fwd": (_I32, [_P] * 6 + [_I64, _I64] + [_I32] * 5 + [_P]),
+    "mg_delta_heads_bwd": (_I32, [_P] * 8 + [_I64, _I64] + [_I32] * 5 + [_P]),
     "mg_delta_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I32, _I32, _I32, _I32]),
     "mg_delta_state_bytes": (_SZ, [_I64, _I64, _I64, _I32, _I32, _I32, _I32]),
     "mg_delta_fwd": (

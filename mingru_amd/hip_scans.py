@@ -1503,6 +1503,54 @@ def delta_scan_impl(Q, K, V, beta, H0, *, chunk_size: int):
                    _delta_tile_chunk(K.shape[3], chunk_size))
 
 
+class _DeltaHeadsFn(torch.autograd.Function):
+    """One joined projection (B, T, N) to the delta kernels' Q, K, V and beta."""
+
+    @staticmethod
+    def forward(ctx, P, H, nh, dk, dv):
+        P = _contig(P, P.dtype)
+        Bn, T, _ = P.shape
+        new = lambda *s: torch.empty(Bn, H, T, *s, dtype=P.dtype, device=P.device)  # noqa: E731
+        Q, K, V, beta = new(dk), new(nh, dk), new(nh, dv), new(nh)
+        nrm = None
+        if any(ctx.needs_input_grad):
+            nrm = torch.empty(Bn, H, T, nh, dtype=torch.float32, device=P.device)
+        dims = (Bn, T, H, nh, dk, dv, 1 if P.dtype == torch.bfloat16 else 0)
+        _call("mg_delta_heads_fwd", _ptr(P), _ptr(Q), _ptr(K), _ptr(V), _ptr(beta), _ptr(nrm),
+              *dims, _stream(P))
+        ctx.save_for_backward(K, beta, nrm)
+        ctx.dims, ctx.shape = dims, P.shape
+        return Q, K, V, beta
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dQ, dK, dV, dbeta):
+        K, beta, nrm = ctx.saved_tensors
+        grads = [_contig(t, K.dtype) for t in (dQ, dK, dV, dbeta)]
+        dP = torch.empty(ctx.shape, dtype=K.dtype, device=K.device)
+        _call("mg_delta_heads_bwd", _ptr(K), _ptr(beta), _ptr(nrm), *(_ptr(t) for t in grads),
+              _ptr(dP), *ctx.dims, _stream(K))
+        return dP, None, None, None, None
+
+
+def delta_heads_impl(P: torch.Tensor, n_heads: int, nh: int, d_k: int, d_v: int):
+    """The delta kernels' ``Q, K, V, beta`` from DeltaMinGRU's joined projection.
+
+    No reference kernel; the arithmetic is the mixer's ``_coeffs`` and layout change
+    (``src/mingru/min_gru.py:3040-3100``): keys L2-normalised, ``beta = 2 sigmoid(.)``.
+    ``P`` (B, T, N) in fp32 or bf16, its rows ``q | k_1 .. k_nh | v_1 .. v_nh | beta_1 ..
+    beta_nh``, each split into heads.  Results in P's dtype; differentiable in ``P``.
+    """
+    N = n_heads * (d_k + nh * (d_k + d_v) + nh)
+    if P.ndim != 3 or P.shape[2] != N or P.numel() == 0:
+        raise ScanFallback(f"joined delta heads: P {tuple(P.shape)}, need (B, T, {N})")
+    if P.dtype not in (torch.float32, torch.bfloat16) or not P.is_cuda:
+        raise ScanFallback(f"joined delta heads need fp32 or bf16 GPU tensors (got {P.dtype})")
+    if max(d_k, d_v) > _DELTA_MAX_DIM:
+        raise ScanFallback(f"joined delta heads need d_k, d_v <= {_DELTA_MAX_DIM}")
+    return _funnel("joined delta heads", _DeltaHeadsFn.apply, P, n_heads, nh, d_k, d_v)
+
+
 # ---------------------------------------------------------------------------
 # DeltaMinGRU decay-gated chunked-WY
 # ---------------------------------------------------------------------------

@@ -1454,17 +1454,40 @@ class DeltaMinGRU(DecayMixin, nn.Module):
             return y, H.reshape(*expected)
         return y
 
+    def _joined_forward(self, x, H, log_gamma=None):
+        """The delta kernels on heads formed from one joined projection, or ``None``
+        (silent in every mode) for the separate projections and their seam, which apply
+        the mode's rules."""
+        linears = (self.linear_q, *self.linear_k, *self.linear_v, *self.linear_beta)
+        backend = _join_backend(x, linears, "delta_heads_impl")
+        if backend is None or max(self.d_k, self.d_v) > _DELTA_AUTO_MAX_DK:
+            return None
+        try:
+            heads = backend.delta_heads_impl(_join_linears(x, linears), self.n_heads, self.nh,
+                                             self.d_k, self.d_v)
+            if log_gamma is None:
+                y, H_T = backend.delta_scan_impl(*heads, H, chunk_size=self.chunk_size)
+            else:
+                y, H_T = backend.delta_gated_scan_impl(*heads, log_gamma, H,
+                                                       chunk_size=self.chunk_size)
+        except backend.ScanFallback:
+            return None
+        return y.permute(0, 2, 1, 3), H_T
+
     def _delta_gated_fused_forward(self, x, H, dt):
         if not _delta_scan_should_try(
             x.is_cuda, T=x.shape[1], chunk_size=self.chunk_size, d_k=self.d_k
         ):
             return None
-        q, ks, vs, betas = self._coeffs(x)
         B, T = dt.shape
         # lambda is per head ("learnable") or one value ("fixed"): (B, n_heads, T) either way.
         log_gamma = (-self._decay_lambda().reshape(1, -1, 1) * dt.unsqueeze(1)).expand(
             B, self.n_heads, T
         )
+        joined = self._joined_forward(x, H, log_gamma)
+        if joined is not None:
+            return joined
+        q, ks, vs, betas = self._coeffs(x)
         return _dispatch_delta_gated_scan(q, ks, vs, betas, log_gamma, H,
                                           chunk_size=self.chunk_size)
 
@@ -1473,6 +1496,9 @@ class DeltaMinGRU(DecayMixin, nn.Module):
             x.is_cuda, T=x.shape[1], chunk_size=self.chunk_size, d_k=self.d_k
         ):
             return None
+        joined = self._joined_forward(x, H)
+        if joined is not None:
+            return joined
         q, ks, vs, betas = self._coeffs(x)
         return _dispatch_delta_scan(q, ks, vs, betas, H, chunk_size=self.chunk_size)
 

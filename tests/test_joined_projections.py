@@ -2,9 +2,11 @@
 the joined form equals the separate one (GPU).
 
 A no-op forward hook on one projection makes a module run its projections separately, so
-the GPU cases compare the two forms of one module.  Both compute the same sums in another
-order: fp32 results agree to about sqrt(K) 2^-24 of the largest term, bf16 ones to bf16's
-2^-8 of each output, doubled where the input's gradient sums separately rounded products.
+the GPU cases compare the two forms of one module.  In fp32 both compute the same sums in
+another order and agree to 2e-5 (sums of up to a few thousand terms at 2^-24 each).  In
+bf16 the separate form rounds after every eager operation and the joined one at its
+kernels' outputs only, so each is held against the module in float64: the joined form may
+be no further off than the separate one, plus one rounding of the output (2^-8).
 """
 
 import copy
@@ -16,7 +18,7 @@ import torch
 from torch import nn
 
 import mingru_amd
-from mingru_amd import MinGRU, SignedMinGRU
+from mingru_amd import DeltaMinGRU, MinGRU, SignedMinGRU
 from mingru_amd import min_gru as mg
 
 BACKEND = "mingru_amd.hip_scans"
@@ -102,6 +104,10 @@ def _pair(cuda, m, dtype):
     return joined, separate
 
 
+def _off(a, b):
+    return ((a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-30)).item()
+
+
 MODULES = [
     # constructor, B, T, time decay
     (lambda: MinGRU(24, 48), 3, 200, False),
@@ -110,6 +116,11 @@ MODULES = [
     (lambda: SignedMinGRU(24, 48), 1, 1, False),
     (lambda: SignedMinGRU(64, 256, coupled=True, learnable_h0=True), 3, 777, False),
     (lambda: SignedMinGRU(32, 520, decay="fixed"), 2, 2100, True),
+    # Head dims of 16-, 32- and 64-lane groups with idle lanes, micro-steps, gated.
+    (lambda: DeltaMinGRU(24, 48, n_heads=4, chunk_size=16), 2, 133, False),
+    (lambda: DeltaMinGRU(40, 96, n_heads=3, nh=2, d_v=20, bias=False), 3, 200, False),
+    (lambda: DeltaMinGRU(64, 192, n_heads=3, nh=2, decay="learnable"), 1, 321, True),
+    (lambda: DeltaMinGRU(32, 100, n_heads=2, d_k=50, d_v=9, decay="fixed"), 2, 140, True),
 ]
 
 
@@ -137,8 +148,17 @@ def test_joined_equals_separate(cuda, case, dtype, monkeypatch):
         res.append([y.detach(), *grads])
     torch.cuda.synchronize()
     assert calls == [1]
-    rel = 2e-5 if dtype == torch.float32 else 2.0**-6
-    for i, (a, b) in enumerate(zip(*res)):
+    if dtype == torch.float32:
+        for i, (a, b) in enumerate(zip(*res)):
+            assert a.dtype == b.dtype and a.shape == b.shape
+            assert _off(a, b) <= 2e-5, f"output {i}: relative difference {_off(a, b):.2e}"
+        return
+    monkeypatch.setenv("MINGRU_SCAN", "eager")
+    ref = copy.deepcopy(joined).double()
+    xi = x.double().requires_grad_()
+    y = ref(xi, delta_t=dt.double()) if decay else ref(xi)
+    exact = [y.detach(), *torch.autograd.grad(y, [xi, *ref.parameters()], gy.double())]
+    for i, (a, b, r) in enumerate(zip(*res, exact)):
         assert a.dtype == b.dtype and a.shape == b.shape
-        off = (a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-30)
-        assert off <= rel, f"output {i}: relative difference {off.item():.2e}"
+        assert _off(a, r) <= 1.5 * _off(b, r) + 2.0**-8, (
+            f"output {i}: joined {_off(a, r):.2e}, separate {_off(b, r):.2e} off float64")
