@@ -390,6 +390,31 @@ int mg_gate_step(int kind, const float* p0, const float* p1, const float* p2, co
 int mg_delta_step(const float* H, const float* q, const float* k, const float* v,
                   const float* beta, const float* log_gamma, float* H_out, float* y, int64_t BH,
                   int nh, int dk, int dv, mg_stream_t stream);
+/* ---- streaming decode of a whole residual block -----------------------------------
+ * No reference kernels: these replace the layer-by-layer MinGRUBlock.step
+ * (src/mingru/min_gru.py:3960-4008) for at most 256 sequences.  dtype (0 fp32, 1 bf16) is
+ * the weights', norms' and block inputs' type; rows of K elements, K a multiple of 4;
+ * ln_w, ln_b (K) NULL together (no LayerNorm), min(B, 16) K floats at most 64 KB with
+ * them.
+ * mg_step_project: out[b] = epi(LN(x[b]) W_s^T + bias_s) for nseg <= 16 projections side by
+ * side (w, bias: nseg pointers, bias entries may be NULL; n: nseg row counts); epi 0 none,
+ * 1 GELU (erf), 2 plus res (B, columns).  x is fp32 if x_f32, out if out_f32. */
+int mg_step_project(int dtype, const void* x, int x_f32, int B, int K, const void* ln_w,
+                    const void* ln_b, float eps, int nseg, const void* const* w,
+                    const void* const* bias, const int* n, int epi, const void* res, void* out,
+                    int out_f32, mg_stream_t stream);
+/* LN(x), the gate projections (kind and their order as mg_gate_step), h = gamma a h_prev +
+ * b and out = x + h.  gamma (B,D) fp32 or NULL; D = K. */
+int mg_step_gate(int dtype, int kind, const void* x, int B, int K, const void* ln_w,
+                 const void* ln_b, float eps, const void* w0, const void* b0, const void* w1,
+                 const void* b1, const void* w2, const void* b2, const float* gamma,
+                 const void* h_prev, void* h, void* out, int D, mg_stream_t stream);
+/* mg_delta_step on raw heads: P (B,N) fp32 rows as mg_delta_heads_fwd's; the key is
+ * normalised and beta formed in the kernel.  H in dtype, y (B,H,dv) fp32. */
+int mg_delta_step_heads(int dtype, const void* H_in, const float* P, const float* log_gamma,
+                        void* H_out, float* y, int64_t B, int H, int nh, int dk, int dv,
+                        mg_stream_t stream);
+
 
 #ifdef __cplusplus
 }

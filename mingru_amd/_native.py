@@ -70,6 +70,14 @@ _SIGNATURES = {
     ),
     "mg_gate_step": (_I32, [_I32] + [_P] * 6 + [_I64, _P]),
     "mg_delta_step": (_I32, [_P] * 8 + [_I64, _I32, _I32, _I32, _P]),
+    "mg_step_project": (
+        _I32,
+        [_I32, _P, _I32, _I32, _I32, _P, _P, _F32, _I32, _P, _P, _P, _I32, _P, _P, _I32, _P],
+    ),
+    "mg_step_gate": (
+        _I32, [_I32, _I32, _P, _I32, _I32, _P, _P, _F32] + [_P] * 10 + [_I32, _P],
+    ),
+    "mg_delta_step_heads": (_I32, [_I32] + [_P] * 5 + [_I64] + [_I32] * 4 + [_P]),
     "mg_log_scan_state_bytes": (_SZ, [_I64, _I64, _I64]),
     "mg_log_scan_fwd": (_I32, [_P, _P, _P, _P, _I64, _I64, _I64, _P, _SZ, _P]),
     "mg_log_scan_bwd": (_I32, [_P] * 7 + [_I64, _I64, _I64, _P, _SZ, _P]),

@@ -41,6 +41,8 @@ __all__ = [
     "gate_scan_packed_impl",
     "gate_step_impl",
     "delta_step_impl",
+    "delta_heads_impl",
+    "block_step_impl",
     "workspace_errors",
     "LookbackError",
 ]
@@ -1715,6 +1717,83 @@ def delta_step_impl(H, q, K, V, beta, log_gamma):
     _call("mg_delta_step", _ptr(h32), _ptr(q32), _ptr(k32), _ptr(v32), _ptr(b32), _ptr(lg32),
           _ptr(Hn), _ptr(y), Bn * nhd, nh, dk, dv, _stream(h32))
     return y.to(q.dtype), Hn.to(H.dtype)
+
+
+# Whole-block decode (csrc/decode_block.hip): sequences per call, sequences a workgroup
+# takes, and the bytes of their normalised inputs it holds.  Each group of 16 sequences
+# reads the weights again and the products run on the vector units, so past a batch times
+# width the library's matrix products are the better ones: three blocks of width 768 take
+# 211 us a token up to 32 sequences (host-bound), 279 at 64 and 507 at 128, layer by layer
+# 760 us of which about 300 are kernels.
+_BLOCK_STEP_MAX_B = 256
+_BLOCK_STEP_MAX_ELEMENTS = 64 * 768
+_BLOCK_STEP_GROUP = 16
+_BLOCK_STEP_MAX_LDS = 64 << 10
+
+
+def _step_project(x, ln, linears, epi: int, res, out, dtype: int) -> None:
+    n = len(linears)
+    K = x.shape[1]
+    pointers = ctypes.c_void_p * n
+    w = pointers(*[p[0].data_ptr() for p in linears])
+    b = pointers(*[None if p[1] is None else p[1].data_ptr() for p in linears])
+    rows = (ctypes.c_int * n)(*[p[0].shape[0] for p in linears])
+    lw, lb, eps = (None, None, 0.0) if ln is None else ln
+    _call("mg_step_project", dtype, _ptr(x), int(x.dtype == torch.float32), x.shape[0], K,
+          _ptr(lw), _ptr(lb), eps, n, w, b, rows, epi, _ptr(res), _ptr(out),
+          int(out.dtype == torch.float32), _stream(x))
+
+
+def block_step_impl(kind: str, x, ln1, proj, h_prev, gamma, delta, ln2, mlp):
+    """One decode step of a residual block; returns ``(x_out, state)``.
+
+    No reference kernel; the arithmetic is ``MinGRUBlock.step``
+    (``src/mingru/min_gru.py:3960-4008``).  ``x`` (B, d); ``ln1``, ``ln2`` are (weight,
+    bias, eps); ``proj`` the mixer's projections as (weight, bias): ``s, z, hpre`` or
+    ``k, hpre`` of the gate kinds, ``q, k.., v.., beta..`` of ``"delta"``, whose ``delta``
+    is (n_heads, nh, d_k, d_v, out_proj).  ``gamma`` is the fp32 decay factor (B, d)
+    (``"delta"``: its log per head, (B, n_heads)) or None.  ``mlp`` is None or the two
+    (weight, bias) pairs.  All tensors share ``x``'s dtype, fp32 or bf16, and are dense.
+    """
+    B, d = x.shape
+    if x.dtype not in (torch.float32, torch.bfloat16) or not 1 <= B <= _BLOCK_STEP_MAX_B:
+        raise ScanFallback(f"block step: {x.dtype} x {tuple(x.shape)}")
+    if d % 4 or B * d > _BLOCK_STEP_MAX_ELEMENTS or 4 * min(B, _BLOCK_STEP_GROUP) * d > _BLOCK_STEP_MAX_LDS:
+        raise ScanFallback(f"block step: width {d} at {B} sequences")
+    pairs = [*proj, *(mlp or ()), *([delta[4]] if delta else ())]
+    ts = [x, h_prev, *ln1[:2], *(t for p in pairs for t in p if t is not None)]
+    if mlp:
+        ts += ln2[:2]
+    dev = x.device
+    for t in ts:
+        if t.dtype != x.dtype or t.device != dev or not t.is_contiguous() or t.data_ptr() % 16:
+            raise ScanFallback("block step needs dense, aligned tensors of one type and device")
+    if dev.type != "cuda" or any(p[0].shape[1] % 4 for p in pairs):
+        raise ScanFallback("block step: GPU tensors with rows of whole 4-element pieces")
+    tag = 1 if x.dtype == torch.bfloat16 else 0
+    mid = torch.empty_like(x)  # x + the mixer's output
+    state = torch.empty_like(h_prev)
+    if kind == "delta":
+        H, nh, dk, dv, out_proj = delta
+        P = torch.empty(B, H * (dk + nh * (dk + dv) + nh), dtype=torch.float32, device=dev)
+        _step_project(x, ln1, proj, 0, None, P, tag)
+        y = torch.empty(B, H * dv, dtype=torch.float32, device=dev)
+        _call("mg_delta_step_heads", tag, _ptr(h_prev), _ptr(P), _ptr(gamma), _ptr(state),
+              _ptr(y), B, H, nh, dk, dv, _stream(x))
+        _step_project(y, None, [out_proj], 2, x, mid, tag)
+    else:
+        (w0, b0), (w1, b1) = proj[:2]
+        w2, b2 = proj[2] if len(proj) == 3 else (None, None)
+        _call("mg_step_gate", tag, GATE_STEP_KINDS[kind], _ptr(x), B, d, _ptr(ln1[0]),
+              _ptr(ln1[1]), ln1[2], _ptr(w0), _ptr(b0), _ptr(w1), _ptr(b1), _ptr(w2), _ptr(b2),
+              _ptr(gamma), _ptr(h_prev), _ptr(state), _ptr(mid), d, _stream(x))
+    if not mlp:
+        return mid, state
+    hidden = torch.empty(B, mlp[0][0].shape[0], dtype=torch.float32, device=dev)
+    _step_project(mid, ln2, mlp[:1], 1, None, hidden, tag)
+    out = torch.empty_like(x)
+    _step_project(hidden, None, mlp[1:], 2, mid, out, tag)
+    return out, state
 
 
 SCAN_IMPLS: dict = {

@@ -333,6 +333,18 @@ def _dispatch_mingru_gate_scan(k: torch.Tensor, hpre: torch.Tensor, log_h0: torc
 _JOIN_MIN_ROWS = 512
 
 
+def _is_plain(m: nn.Module, cls: type) -> bool:
+    """Whether calling ``m`` computes what ``cls.forward`` does on its parameters and
+    nothing else: no subclass, hook, replaced forward or parameter of another kind."""
+    return (
+        type(m) is cls
+        and "forward" not in m.__dict__
+        and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                 or m._backward_pre_hooks)
+        and all(p is None or type(p) is nn.Parameter for p in m._parameters.values())
+    )
+
+
 def _join_backend(x: torch.Tensor, linears, impl: str):
     """The backend, if it has ``impl`` and one joined projection of ``x`` may stand in for
     ``linears``; else ``None``.
@@ -354,13 +366,9 @@ def _join_backend(x: torch.Tensor, linears, impl: str):
         return None
     like = None
     for m in linears:
-        if type(m) is not nn.Linear or "forward" in m.__dict__ or (
-            m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-        ):
+        if not _is_plain(m, nn.Linear):
             return None
         w, b = m.weight, m.bias
-        if type(w) is not nn.Parameter or not (b is None or type(b) is nn.Parameter):
-            return None
         this = (w.dtype, w.device, w.requires_grad,
                 None if b is None else (b.dtype, b.device, b.requires_grad))
         if like is not None and this != like:
@@ -429,6 +437,102 @@ def _dispatch_step(what: str, is_cuda: bool, call):
         )
         _warned_step_fallback = True
     return None
+
+
+def _block_step_plan(block: nn.Module):
+    """``block``'s step as ``block_step_impl`` takes it, ``(kind, ln1, proj, delta, ln2,
+    mlp)``, or ``None`` where it has a part the fused step does not stand in for."""
+    mixer, norm1 = block.mingru, block.norm1
+    kind = {MinGRU: "mingru", SignedMinGRU: "signed", DeltaMinGRU: "delta"}.get(type(mixer))
+    if kind is None or block.training and block.drop.p > 0:
+        return None
+    delta = None
+    if kind == "mingru":
+        linears = (mixer.linear_z, mixer.linear_h)
+    elif kind == "signed":
+        linears = (mixer.linear_s, mixer.linear_z, mixer.linear_h)
+        kind = "signed_coupled" if mixer.coupled else "signed"
+    else:
+        linears = (mixer.linear_q, *mixer.linear_k, *mixer.linear_v, *mixer.linear_beta)
+        if len(linears) > 16 or max(mixer.d_k, mixer.d_v) > _DELTA_AUTO_MAX_DK:
+            return None
+        out = mixer.out_proj
+        if not _is_plain(out, nn.Linear):
+            return None
+        delta = (mixer.n_heads, mixer.nh, mixer.d_k, mixer.d_v, (out.weight, out.bias))
+    norms, mlp = [norm1], None
+    if block.mlp is not None:
+        seq = block.mlp
+        if not (_is_plain(seq, nn.Sequential) and len(seq) == 4 and _is_plain(seq[1], nn.GELU)
+                and seq[1].approximate == "none" and _is_plain(seq[2], nn.Dropout)
+                and _is_plain(seq[0], nn.Linear) and _is_plain(seq[3], nn.Linear)):
+            return None
+        norms.append(block.norm2)
+        mlp = ((seq[0].weight, seq[0].bias), (seq[3].weight, seq[3].bias))
+    for m in norms:
+        if not _is_plain(m, nn.LayerNorm) or m.weight is None or m.bias is None:
+            return None
+    if not all(_is_plain(m, nn.Linear) for m in linears):
+        return None
+    ln = [(m.weight, m.bias, m.eps) for m in norms]
+    return (kind, ln[0], [(m.weight, m.bias) for m in linears], delta,
+            ln[1] if mlp else None, mlp)
+
+
+def _dispatch_block_step(block: nn.Module, x_t, h_prev, delta_t):
+    """A whole residual block's decode step in a few launches, or ``None`` (silent in
+    every mode) for the layer-by-layer step, whose seams apply the mode's rules."""
+    if (_resolve_scan_mode(x_t.is_cuda) is None or x_t.dim() != 2
+            or torch.is_autocast_enabled() or torch.nn.modules.module._has_any_global_hook()):
+        return None
+    try:
+        from mingru_amd import hip_scans as backend
+    except ImportError:
+        return None
+    if not hasattr(backend, "block_step_impl") or backend.available() is not True:
+        return None
+    plan = _block_step_plan(block)
+    if plan is None:
+        return None
+    kind, ln1, proj, delta, ln2, mlp = plan
+    mixer, B = block.mingru, x_t.size(0)
+    if x_t.size(1) != ln1[0].numel() or mixer.hidden_size != x_t.size(1):
+        return None
+    dt = mixer._prepare_decay(delta_t, canonical_ndim=1)
+    if dt is not None and tuple(dt.shape) != (B,):
+        return None
+    gamma = None
+    if kind == "delta":
+        width = mixer.n_heads * mixer.d_k * mixer.d_v
+        if dt is not None:
+            gamma = (-mixer._decay_lambda() * dt.unsqueeze(-1)).expand(B, mixer.n_heads)
+    else:
+        width = mixer.hidden_size
+        if dt is not None:
+            gamma = mixer._decay_gamma(dt).expand(B, width)
+    if gamma is not None:
+        gamma = gamma.to(torch.float32).contiguous()
+    if h_prev is None:
+        h_prev = _default_step_state(mixer, x_t, width)
+    elif tuple(h_prev.shape) != (B, width):
+        return None
+    try:
+        return backend.block_step_impl(kind, x_t, ln1, proj, h_prev, gamma, delta, ln2, mlp)
+    except (backend.ScanFallback, RuntimeError):
+        return None
+
+
+def _default_step_state(mixer, x_t, width):
+    """The state ``mixer.step`` starts from when it is given none, dense."""
+    if isinstance(mixer, MinGRU):
+        if mixer.h0_pre is None:
+            return x_t.new_full((x_t.size(0), width), 0.5)
+        h = g(mixer.h0_pre)[:, 0]
+    elif isinstance(mixer, SignedMinGRU) and mixer.h0 is not None:
+        h = mixer.h0[:, 0]
+    else:
+        return x_t.new_zeros(x_t.size(0), width)
+    return h.expand(x_t.size(0), width).contiguous()
 
 
 def _dispatch_gate_step(kind: str, p0, p1, p2, gamma, h_prev):
@@ -1711,6 +1815,9 @@ class MinGRUBlock(nn.Module):
     @torch.no_grad()
     def step(self, x_t, h_prev, delta_t=None):
         delta_t = _match_delta_t_dtype(delta_t, self.mingru)
+        fused = _dispatch_block_step(self, x_t, h_prev, delta_t)
+        if fused is not None:
+            return fused
         if getattr(self.mingru, "carries_matrix_state", False):
             y_t, state = self.mingru.step(self.norm1(x_t), h_prev, delta_t)
         else:
