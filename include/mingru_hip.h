@@ -235,6 +235,17 @@ int mg_angle_scan_gated_bwd(const float* theta, const float* u, const float* gam
                             float* dgamma, float* dz, float* dhpre, float* dh0, int64_t B,
                             int64_t T, int64_t n, int k, int rounds, int flags, void* ws,
                             size_t ws_bytes, mg_stream_t stream);
+/* The gated form on one joined projection, 8x8 blocks: P (B,T,n (16 + 4 rounds)), rows
+ * z (n,8) | hpre (n,8) | theta (n,rounds,4) -> h (B,T,n,8); the backward writes P's whole
+ * gradient.  gamma (B,T,n) or NULL (no decay; then dgamma too).  Workspace and state as
+ * mg_angle_scan_gated_*. */
+int mg_angle_scan_joined_fwd(const float* P, const float* gamma, const float* h0, float* h,
+                             float* chunk_prod, int64_t B, int64_t T, int64_t n, int rounds,
+                             void* ws, size_t ws_bytes, mg_stream_t stream);
+int mg_angle_scan_joined_bwd(const float* P, const float* gamma, const float* h0, const float* h,
+                             const float* chunk_prod, const float* gh, float* dP, float* dgamma,
+                             float* dh0, int64_t B, int64_t T, int64_t n, int rounds, void* ws,
+                             size_t ws_bytes, mg_stream_t stream);
 
 /* ---- angle-fused scan driven by run-time plane tables -------------------------
  * Replaces the same reference kernels as mg_angle_scan_fwd/bwd

@@ -97,6 +97,8 @@ _SIGNATURES = {
     "mg_angle_scan_gated_bwd": (
         _I32, [_P] * 15 + [_I64, _I64, _I64, _I32, _I32, _I32, _P, _SZ, _P],
     ),
+    "mg_angle_scan_joined_fwd": (_I32, [_P] * 5 + [_I64, _I64, _I64, _I32, _P, _SZ, _P]),
+    "mg_angle_scan_joined_bwd": (_I32, [_P] * 9 + [_I64, _I64, _I64, _I32, _P, _SZ, _P]),
     "mg_angle_scan_tables_state_bytes": (_SZ, [_I64, _I64, _I64, _I32]),
     "mg_angle_scan_tables_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I32]),
     "mg_angle_scan_tables_fwd": (

@@ -338,6 +338,13 @@ struct AnArgs {
   float* dhpre;
   int rounds;
   int na;  // angles per token
+  // Joined heads (GP): theta, z and hpre are slices of one projection's rows, so a token's
+  // planes lie a whole row apart: xth and xk are a row's elements beyond the tensor's own
+  // (n na and n K), for theta and dtheta, and for z, hpre and their gradients.  0: dense.
+  // The four token passes take as long either way; the layer around them runs one product
+  // each way instead of three (GivensMinGRU fp32, B=8, T=2048, 512 wide: 1081 -> 875 us a
+  // step, 750 of them in the products).
+  int64_t xth, xk;
 };
 
 // The per-token scale and input of the brick-wall kernels, plain or through the gated
@@ -349,11 +356,12 @@ __device__ __forceinline__ float an_scale(const AnArgs& a, int64_t lane_tok) {
 }
 
 template <int K, bool GP>
-__device__ __forceinline__ void an_input(const AnArgs& a, int64_t lane_tok, float (&bt)[K]) {
+__device__ __forceinline__ void an_input(const AnArgs& a, int64_t lane_tok, int64_t tok,
+                                         float (&bt)[K]) {
   if constexpr (GP) {
     float zz[K], hp[K];
-    ld<K>(zz, a.b + lane_tok * K);
-    ld<K>(hp, a.hpre + lane_tok * K);
+    ld<K>(zz, a.b + lane_tok * K + tok * a.xk);
+    ld<K>(hp, a.hpre + lane_tok * K + tok * a.xk);
 #pragma unroll
     for (int i = 0; i < K; ++i) bt[i] = mg_sigmoid(zz[i]) * hp[i];
   } else {
@@ -364,20 +372,20 @@ __device__ __forceinline__ void an_input(const AnArgs& a, int64_t lane_tok, floa
 // db_t = dL/dh_t (the token's adjoint) stored, or through the gated prologue dL/dz
 // and dL/dhpre.
 template <int K, bool GP>
-__device__ __forceinline__ void an_store_db(const AnArgs& a, int64_t lane_tok,
+__device__ __forceinline__ void an_store_db(const AnArgs& a, int64_t lane_tok, int64_t tok,
                                             const float (&gt)[K]) {
   if constexpr (GP) {
     float zz[K], hp[K], dz[K], dh[K];
-    ld<K>(zz, a.b + lane_tok * K);
-    ld<K>(hp, a.hpre + lane_tok * K);
+    ld<K>(zz, a.b + lane_tok * K + tok * a.xk);
+    ld<K>(hp, a.hpre + lane_tok * K + tok * a.xk);
 #pragma unroll
     for (int i = 0; i < K; ++i) {
       const float sg = mg_sigmoid(zz[i]);
       dh[i] = gt[i] * sg;
       dz[i] = dh[i] * hp[i] * (1.f - sg);
     }
-    st<K>(a.out + lane_tok * K, dz);
-    st<K>(a.dhpre + lane_tok * K, dh);
+    st<K>(a.out + lane_tok * K + tok * a.xk, dz);
+    st<K>(a.dhpre + lane_tok * K + tok * a.xk, dh);
   } else {
     st<K>(a.out + lane_tok * K, gt);
   }
@@ -395,7 +403,7 @@ __device__ __forceinline__ void an_input_reg(const float (&v)[K], const float (&
 }
 
 template <int K, bool GP>
-__device__ __forceinline__ void an_store_db_reg(const AnArgs& a, int64_t lane_tok,
+__device__ __forceinline__ void an_store_db_reg(const AnArgs& a, int64_t lane_tok, int64_t tok,
                                                 const float (&gt)[K], const float (&zz)[GP ? K : 1],
                                                 const float (&hp)[GP ? K : 1]) {
   if constexpr (GP) {
@@ -406,8 +414,8 @@ __device__ __forceinline__ void an_store_db_reg(const AnArgs& a, int64_t lane_to
       dh[i] = gt[i] * sg;
       dz[i] = dh[i] * hp[i] * (1.f - sg);
     }
-    st<K>(a.out + lane_tok * K, dz);
-    st<K>(a.dhpre + lane_tok * K, dh);
+    st<K>(a.out + lane_tok * K + tok * a.xk, dz);
+    st<K>(a.dhpre + lane_tok * K + tok * a.xk, dh);
   } else {
     st<K>(a.out + lane_tok * K, gt);
   }
@@ -452,14 +460,17 @@ struct BrickTok {
   float hp[HP ? K : 1];
   float d, gm;  // the scale input (u under the gated prologue) and the decay
 
-  __device__ __forceinline__ void load(const AnArgs& a, const float* vec, int64_t lane_tok,
-                                       int64_t t, int64_t n, int64_t blk) {
-    const float* th = a.theta + lane_tok * (R * H);
+  // xvec: vec's elements per token beyond its own (a.xk for z, 0 for dense tensors).
+  __device__ __forceinline__ void load(const AnArgs& a, const float* vec, int64_t xvec,
+                                       int64_t tok, int64_t plane, int64_t t, int64_t n,
+                                       int64_t blk) {
+    const int64_t lane_tok = tok * n + plane;
+    const float* th = a.theta + lane_tok * (R * H) + tok * a.xth;
 #pragma unroll
     for (int r = 0; r < R; ++r) ld<H>(ang[r], th + r * H);
-    ld<K>(v, vec + lane_tok * K);
-    if constexpr (HQ) ld<K>(hq, a.hpre + lane_tok * K);
-    if constexpr (ZB) ld<K>(zb, a.b + lane_tok * K);
+    ld<K>(v, vec + lane_tok * K + tok * xvec);
+    if constexpr (HQ) ld<K>(hq, a.hpre + lane_tok * K + tok * a.xk);
+    if constexpr (ZB) ld<K>(zb, a.b + lane_tok * K + tok * a.xk);
     d = HS ? a.scale[lane_tok] : 1.f;
     gm = HD ? a.gamma[lane_tok] : 1.f;
     if constexpr (HP) {
@@ -705,7 +716,7 @@ __global__ __launch_bounds__(AN_RED_THREADS) void angle_fwd_reduce(AnArgs a, AnG
             token_pairs<Tok>(
                 t0, (int)(te - t0), 1,
                 [&](Tok& k, int64_t t) {
-                  k.load(a, a.b, (th.bb * g.T + t) * g.n + th.plane, t, g.n, th.blk);
+                  k.load(a, a.b, a.xk, th.bb * g.T + t, th.plane, t, g.n, th.blk);
                 },
                 [&](const Tok& cur, int64_t) {
                   const float d = HS ? (GP ? mg_tanh(cur.d) : cur.d) : 1.f;
@@ -719,13 +730,13 @@ __global__ __launch_bounds__(AN_RED_THREADS) void angle_fwd_reduce(AnArgs a, AnG
                 });
           } else {
             for (int64_t t = t0; t < te; ++t) {
-              const int64_t lane_tok = (th.bb * g.T + t) * g.n + th.plane;
+              const int64_t tok = th.bb * g.T + t, lane_tok = tok * g.n + th.plane;
               const float d = HS ? an_scale<GP>(a, lane_tok) : 1.f;
               const float gm = HD ? a.gamma[lane_tok] : 1.f;
-              apply_M<K, SCHED, HS, false, K + 1>(X, a.theta + lane_tok * a.na, a.rounds, d, 1.f);
+              apply_M<K, SCHED, HS, false, K + 1>(X, a.theta + lane_tok * a.na + tok * a.xth, a.rounds, d, 1.f);
               if (HD) gprod *= gm;
               float bt[K];
-              an_input<K, GP>(a, lane_tok, bt);
+              an_input<K, GP>(a, lane_tok, tok, bt);
 #pragma unroll
               for (int i = 0; i < K; ++i)
                 X[i][K] = HD ? fmaf(gm, X[i][K], bt[i]) : X[i][K] + bt[i];
@@ -981,7 +992,7 @@ __global__ __launch_bounds__(MG_WAVE* AN_WAVES) void angle_fwd_final(AnArgs a, A
           k.template load<false>(a, a.b, (th.bb * g.T + t) * g.n + th.plane, t, g.n, th.blk);
         },
         [&](const Tok& cur, int64_t t) {
-          const int64_t lane_tok = (th.bb * g.T + t) * g.n + th.plane;
+          const int64_t tok = th.bb * g.T + t, lane_tok = tok * g.n + th.plane;
           apply_M_lex<K, HS, HD, 1>(v, cur.ang, cur.d, cur.gm);
           float bt[K];
 #pragma unroll
@@ -999,10 +1010,10 @@ __global__ __launch_bounds__(MG_WAVE* AN_WAVES) void angle_fwd_final(AnArgs a, A
         token_pairs<Tok>(
             t0, (int)(te - t0), 1,
             [&](Tok& k, int64_t t) {
-              k.load(a, a.b, (th.bb * g.T + t) * g.n + th.plane, t, g.n, th.blk);
+              k.load(a, a.b, a.xk, th.bb * g.T + t, th.plane, t, g.n, th.blk);
             },
             [&](const Tok& cur, int64_t t) {
-              const int64_t lane_tok = (th.bb * g.T + t) * g.n + th.plane;
+              const int64_t tok = th.bb * g.T + t, lane_tok = tok * g.n + th.plane;
               const float d = HS ? (GP ? mg_tanh(cur.d) : cur.d) : 1.f;
               apply_M_brick<K, R, HS, HD, 1>(v, cur.ang, d, cur.gm);
               float bt[K];
@@ -1016,12 +1027,12 @@ __global__ __launch_bounds__(MG_WAVE* AN_WAVES) void angle_fwd_final(AnArgs a, A
             });
       } else {
         for (int64_t t = t0; t < te; ++t) {
-          const int64_t lane_tok = (th.bb * g.T + t) * g.n + th.plane;
+          const int64_t tok = th.bb * g.T + t, lane_tok = tok * g.n + th.plane;
           const float d = HS ? an_scale<GP>(a, lane_tok) : 1.f;
           const float gm = HD ? a.gamma[lane_tok] : 1.f;
-          apply_M<K, SCHED, HS, HD, 1>(v, a.theta + lane_tok * a.na, a.rounds, d, gm);
+          apply_M<K, SCHED, HS, HD, 1>(v, a.theta + lane_tok * a.na + tok * a.xth, a.rounds, d, gm);
           float bt[K];
-          an_input<K, GP>(a, lane_tok, bt);
+          an_input<K, GP>(a, lane_tok, tok, bt);
 #pragma unroll
           for (int i = 0; i < K; ++i) {
             v[i][0] += bt[i];
@@ -1249,7 +1260,7 @@ __global__ __launch_bounds__(MG_WAVE* AN_WAVES) void angle_bwd_reduce(AnArgs a, 
         token_pairs<Tok>(
             te - 1, (int)(te - t0), -1,
             [&](Tok& k, int64_t t) {
-              k.load(a, a.gh, (th.bb * g.T + t) * g.n + th.plane, t, g.n, th.blk);
+              k.load(a, a.gh, 0, th.bb * g.T + t, th.plane, t, g.n, th.blk);
             },
             [&](const Tok& cur, int64_t) {
               const float d = HS ? (GP ? mg_tanh(cur.d) : cur.d) : 1.f;
@@ -1259,14 +1270,14 @@ __global__ __launch_bounds__(MG_WAVE* AN_WAVES) void angle_bwd_reduce(AnArgs a, 
             });
       } else {
         for (int64_t t = te - 1; t >= t0; --t) {
-          const int64_t lane_tok = (th.bb * g.T + t) * g.n + th.plane;
+          const int64_t tok = th.bb * g.T + t, lane_tok = tok * g.n + th.plane;
           const float d = HS ? an_scale<GP>(a, lane_tok) : 1.f;
           const float gm = HD ? a.gamma[lane_tok] : 1.f;
           float gt[K];
           ld<K>(gt, a.gh + lane_tok * K);
 #pragma unroll
           for (int i = 0; i < K; ++i) x[i][0] += gt[i];
-          apply_Mt<K, SCHED, HS, HD, 1>(x, a.theta + lane_tok * a.na, a.rounds, d, gm);
+          apply_Mt<K, SCHED, HS, HD, 1>(x, a.theta + lane_tok * a.na + tok * a.xth, a.rounds, d, gm);
         }
       }
     });
@@ -1564,7 +1575,7 @@ __global__ __launch_bounds__(MG_WAVE* AN_WAVES) void angle_bwd_final(AnArgs a, A
           k.template load<true>(a, a.gh, (th.bb * g.T + t) * g.n + th.plane, t, g.n, th.blk);
         },
         [&](const Tok& cur, int64_t t) {
-          const int64_t lane_tok = (th.bb * g.T + t) * g.n + th.plane;
+          const int64_t tok = th.bb * g.T + t, lane_tok = tok * g.n + th.plane;
           float gt[K];
 #pragma unroll
           for (int i = 0; i < K; ++i) {
@@ -1599,10 +1610,10 @@ __global__ __launch_bounds__(MG_WAVE* AN_WAVES) void angle_bwd_final(AnArgs a, A
         token_pairs<Tok>(
             te - 1, (int)(te - t0), -1,
             [&](Tok& k, int64_t t) {
-              k.load(a, a.gh, (th.bb * g.T + t) * g.n + th.plane, t, g.n, th.blk);
+              k.load(a, a.gh, 0, th.bb * g.T + t, th.plane, t, g.n, th.blk);
             },
             [&](const Tok& cur, int64_t t) {
-              const int64_t lane_tok = (th.bb * g.T + t) * g.n + th.plane;
+              const int64_t tok = th.bb * g.T + t, lane_tok = tok * g.n + th.plane;
               const float d = HS ? (GP ? mg_tanh(cur.d) : cur.d) : 1.f;
               float gt[K];
 #pragma unroll
@@ -1610,21 +1621,22 @@ __global__ __launch_bounds__(MG_WAVE* AN_WAVES) void angle_bwd_final(AnArgs a, A
                 y[i][0] += cur.v[i];
                 gt[i] = y[i][0];
               }
-              an_store_db_reg<K, GP>(a, lane_tok, gt, cur.zb, cur.hq);  // db_t (or dz, dhpre)
+              an_store_db_reg<K, GP>(a, lane_tok, tok, gt, cur.zb, cur.hq);  // db_t (or dz, dhpre)
               float dd = 0.f, dg = 0.f, gr[NA];
               token_grad_brick<K, R, HS, HD>(y, cur.hp, cur.ang, gr, d, cur.gm, dd, dg);
               if constexpr (NA % 4 == 0) {
-                if (whole) wave_rows_store<NA>(a.dtheta + (lane_tok - lane) * NA, gr, rows, lane);
-                else st<NA>(a.dtheta + lane_tok * NA, gr);
-              } else {
-                st<NA>(a.dtheta + lane_tok * NA, gr);  // partial-line rows: the L2 merges them
+                float* dth = a.dtheta + tok * a.xth;
+                if (whole) wave_rows_store<NA>(dth + (lane_tok - lane) * NA, gr, rows, lane);
+                else st<NA>(dth + lane_tok * NA, gr);
+              } else {  // partial-line rows: the L2 merges them
+                st<NA>(a.dtheta + lane_tok * NA + tok * a.xth, gr);
               }
               if (HS) a.dscale[lane_tok] = GP ? dd * (1.f - d * d) : dd;  // GP: dL/du, d = tanh(u)
               if (HD) a.dgamma[lane_tok] = dg;
             });
       } else {
         for (int64_t t = te - 1; t >= t0; --t) {
-          const int64_t lane_tok = (th.bb * g.T + t) * g.n + th.plane;
+          const int64_t tok = th.bb * g.T + t, lane_tok = tok * g.n + th.plane;
           const float d = HS ? an_scale<GP>(a, lane_tok) : 1.f;
           const float gm = HD ? a.gamma[lane_tok] : 1.f;
           float gt[K], hp[K];
@@ -1636,10 +1648,10 @@ __global__ __launch_bounds__(MG_WAVE* AN_WAVES) void angle_bwd_final(AnArgs a, A
             y[i][0] += gt[i];
             gt[i] = y[i][0];
           }
-          an_store_db<K, GP>(a, lane_tok, gt);  // db_t = dL/dh_t (or dz, dhpre)
+          an_store_db<K, GP>(a, lane_tok, tok, gt);  // db_t = dL/dh_t (or dz, dhpre)
           float dd = 0.f, dg = 0.f;
-          token_grad<K, SCHED, HS, HD>(y, hp, a.theta + lane_tok * a.na,
-                                       a.dtheta + lane_tok * a.na, a.rounds, d, gm, dd, dg);
+          token_grad<K, SCHED, HS, HD>(y, hp, a.theta + lane_tok * a.na + tok * a.xth,
+                                       a.dtheta + lane_tok * a.na + tok * a.xth, a.rounds, d, gm, dd, dg);
           if (HS) a.dscale[lane_tok] = GP ? dd * (1.f - d * d) : dd;  // GP: dL/du, d = tanh(u)
           if (HD) a.dgamma[lane_tok] = dg;
         }
@@ -1802,6 +1814,19 @@ bool an_geometry_ok(int64_t B, int64_t T, int64_t n) {
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
+// The heads of one joined projection, 8x8 blocks: rows z (n, 8) | hpre (n, 8) |
+// theta (n, rounds, 4).  Every slice starts at a multiple of 4 floats.
+void an_joined(AnArgs& a, const float* P, int64_t n, int rounds) {
+  a.rounds = rounds;
+  a.na = rounds * 4;
+  a.b = P;
+  a.hpre = P + n * 8;
+  a.theta = P + 2 * n * 8;
+  const int64_t row = n * (16 + a.na);
+  a.xk = row - n * 8;
+  a.xth = row - n * a.na;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1929,6 +1954,46 @@ int mg_angle_scan_gated_bwd(const float* theta, const float* u, const float* gam
   a.na = rounds * (k / 2);
   return an_dispatch<true>(a, B, T, n, k, SCHED_BRICK, flags | AN_FLAG_GATED, ws, ws_bytes,
                            stream);
+}
+
+int mg_angle_scan_joined_fwd(const float* P, const float* gamma, const float* h0, float* h,
+                             float* chunk_prod, int64_t B, int64_t T, int64_t n, int rounds,
+                             void* ws, size_t ws_bytes, hipStream_t stream) {
+  if (!P || !h0 || !h || !chunk_prod || !ws || !an_args_ok(B, T, n, 8, SCHED_BRICK, rounds) ||
+      !an_geometry_ok(B, T, n) || !aligned16(P) || !aligned16(h0) || !aligned16(h))
+    return MG_ERR_ARG;
+  AnArgs a{};
+  an_joined(a, P, n, rounds);
+  a.gamma = gamma;
+  a.h0 = h0;
+  a.out = h;
+  a.prod = chunk_prod;
+  return an_dispatch<false>(a, B, T, n, 8, SCHED_BRICK, (gamma ? 2 : 0) | AN_FLAG_GATED, ws,
+                            ws_bytes, stream);
+}
+
+int mg_angle_scan_joined_bwd(const float* P, const float* gamma, const float* h0, const float* h,
+                             const float* chunk_prod, const float* gh, float* dP, float* dgamma,
+                             float* dh0, int64_t B, int64_t T, int64_t n, int rounds, void* ws,
+                             size_t ws_bytes, hipStream_t stream) {
+  if (!P || !h0 || !h || !chunk_prod || !gh || !dP || !dh0 || !ws || !gamma != !dgamma ||
+      !an_args_ok(B, T, n, 8, SCHED_BRICK, rounds) || !an_geometry_ok(B, T, n) || !aligned16(P) ||
+      !aligned16(h0) || !aligned16(h) || !aligned16(gh) || !aligned16(dP) || !aligned16(dh0))
+    return MG_ERR_ARG;
+  AnArgs a{};
+  an_joined(a, P, n, rounds);
+  a.gamma = gamma;
+  a.h0 = h0;
+  a.h = h;
+  a.gh = gh;
+  a.out = dP;
+  a.dhpre = dP + n * 8;
+  a.dtheta = dP + 2 * n * 8;
+  a.dgamma = dgamma;
+  a.dh0 = dh0;
+  a.prod = const_cast<float*>(chunk_prod);
+  return an_dispatch<true>(a, B, T, n, 8, SCHED_BRICK, (gamma ? 2 : 0) | AN_FLAG_GATED, ws,
+                           ws_bytes, stream);
 }
 
 }  // extern "C"

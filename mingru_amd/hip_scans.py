@@ -41,6 +41,7 @@ __all__ = [
     "gate_scan_packed_impl",
     "gate_step_impl",
     "delta_step_impl",
+    "angle_joined_scan_impl",
     "delta_heads_impl",
     "block_step_impl",
     "workspace_errors",
@@ -1351,6 +1352,55 @@ def angle_gated_scan_impl(theta, u, gamma, z, hpre, h0, perm, sgn, p2p, *, has_s
     return _funnel("angle-fused (gated heads)", _AngleGatedFn.apply, theta,
                    u if has_scale else None, gamma if has_decay else None, z, hpre, h0, rounds,
                    flags)
+
+
+class _JoinedAngleGatedFn(torch.autograd.Function):
+    """``_AngleGatedFn`` (8x8 blocks, no scale) on one joined projection (B, T, N)."""
+
+    @staticmethod
+    def forward(ctx, P, gamma, h0, rounds):
+        P, h032 = _as_f32(P, h0)
+        gm = _as_f32(gamma)[0] if gamma is not None else None
+        Bn, T, _ = P.shape
+        n = h032.shape[1]
+        dims = (Bn, T, n, rounds)
+        h = torch.empty(Bn, T, n, 8, dtype=torch.float32, device=P.device)
+        prod = torch.empty(max(_size("mg_angle_scan_state_bytes", Bn, T, n, 8), 16) // 4,
+                           dtype=torch.float32, device=P.device)
+        ws = _workspace(_size("mg_angle_scan_workspace_bytes", Bn, T, n, 8), P.device)
+        _call("mg_angle_scan_joined_fwd", _ptr(P), _ptr(gm), _ptr(h032), _ptr(h), _ptr(prod),
+              *dims, _ptr(ws), ws.numel(), _stream(P))
+        ctx.save_for_backward(P, gm, h032, h, prod)
+        ctx.meta = (dims, None if gamma is None else gamma.dtype, h0.dtype)
+        return h
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, gh):
+        P, gm, h032, h, prod = ctx.saved_tensors
+        dims, gdt, h0dt = ctx.meta
+        (gh32,) = _as_f32(gh)
+        dP, dh0 = torch.empty_like(P), torch.empty_like(h032)
+        dgm = torch.empty_like(gm) if gm is not None else None
+        ws = _workspace(_size("mg_angle_scan_workspace_bytes", *dims[:3], 8), h.device)
+        _call("mg_angle_scan_joined_bwd", _ptr(P), _ptr(gm), _ptr(h032), _ptr(h), _ptr(prod),
+              _ptr(gh32), _ptr(dP), _ptr(dgm), _ptr(dh0), *dims, _ptr(ws), ws.numel(), _stream(h))
+        return dP, None if dgm is None else dgm.to(gdt), dh0.to(h0dt), None
+
+
+def angle_joined_scan_impl(P, gamma, h0, rounds: int):
+    """``angle_gated_scan_impl`` for GivensMinGRU's 8x8 brick-wall blocks on one joined
+    fp32 projection: ``P`` (B, T, n (16 + 4 rounds)), its rows ``z | hpre | theta``;
+    ``gamma`` (B, T, n) or None, ``h0`` (B, n, 8).  Returns ``h`` (B, T, n, 8)."""
+    if P.ndim != 3 or h0.ndim != 3 or h0.shape[2] != 8 or P.dtype != torch.float32:
+        raise ScanFallback(f"joined angle scan: P {tuple(P.shape)} {P.dtype}")
+    Bn, T, N = P.shape
+    n = h0.shape[1]
+    if (N != n * (16 + 4 * rounds) or h0.shape[0] != Bn or not 1 <= rounds <= _ANGLE_MAX_ROT
+            or P.numel() == 0 or (gamma is not None and tuple(gamma.shape) != (Bn, T, n))):
+        raise ScanFallback(f"joined angle scan: P {tuple(P.shape)}, h0 {tuple(h0.shape)}")
+    _same_device(P, h0, *([] if gamma is None else [gamma]))
+    return _funnel("joined angle scan", _JoinedAngleGatedFn.apply, P, gamma, h0, rounds)
 
 
 # ---------------------------------------------------------------------------

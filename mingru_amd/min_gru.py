@@ -444,7 +444,7 @@ def _block_step_plan(block: nn.Module):
     mlp)``, or ``None`` where it has a part the fused step does not stand in for."""
     mixer, norm1 = block.mingru, block.norm1
     kind = {MinGRU: "mingru", SignedMinGRU: "signed", DeltaMinGRU: "delta"}.get(type(mixer))
-    if kind is None or block.training and block.drop.p > 0:
+    if kind is None:
         return None
     delta = None
     if kind == "mingru":
@@ -465,6 +465,7 @@ def _block_step_plan(block: nn.Module):
         seq = block.mlp
         if not (_is_plain(seq, nn.Sequential) and len(seq) == 4 and _is_plain(seq[1], nn.GELU)
                 and seq[1].approximate == "none" and _is_plain(seq[2], nn.Dropout)
+                and not (seq[2].training and seq[2].p > 0)
                 and _is_plain(seq[0], nn.Linear) and _is_plain(seq[3], nn.Linear)):
             return None
         norms.append(block.norm2)
@@ -1364,11 +1365,32 @@ class GivensMinGRU(DecayMixin, nn.Module):
         scale = torch.ones(B, T, n, dtype=x.dtype, device=x.device)
         return theta, scale, gamma, b
 
+    def _joined_forward(self, x, h0_blocks, dt):
+        """The gated angle scan from one joined projection (8x8 blocks, fp32), or ``None``
+        (silent in every mode) for the separate projections and their seams."""
+        linears = (self.linear_z, self.linear_h, self.linear_theta)
+        if (self.k != 8 or x.dim() != 3 or x.numel() == 0 or torch.is_autocast_enabled()
+                or self.linear_z.weight.dtype != torch.float32):
+            return None
+        backend = _join_backend(x, linears, "angle_joined_scan_impl")
+        if backend is None:
+            return None
+        B, T, _ = x.shape
+        gamma = self._decay_gamma(dt).expand(B, T, self.n_blocks) if dt is not None else None
+        try:
+            return backend.angle_joined_scan_impl(_join_linears(x, linears), gamma, h0_blocks,
+                                                  self.rounds)
+        except backend.ScanFallback:
+            return None
+
     def _angle_fused_forward(self, x, h0_blocks, dt):
         if not _angle_scan_should_try(x.is_cuda):
             return None
         B, T, _ = x.shape
         n, k, R = self.n_blocks, self.k, self.rounds
+        h = self._joined_forward(x, h0_blocks, dt)
+        if h is not None:
+            return h.reshape(B, T, self.hidden_size)
         perm, sgn, p2p = self._angle_plane_meta(x.device)
         # The sigmoid(z) * h~ input formed in the kernel (brick-wall k <= 8).
         gamma = self._decay_gamma(dt).expand(B, T, n) if dt is not None else None
