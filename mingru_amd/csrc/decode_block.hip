@@ -237,7 +237,7 @@ __global__ __launch_bounds__(MG_WAVE) void delta_step_heads(const E* __restrict_
     float k = pk[mh * dk + jk];
     k = j < dk ? k : 0.f;
     k /= fmaxf(sqrtf(mg_group_sum<64>(k * k)), 1e-12f);
-    const float beta = 2.f * mg_sigmoid(pb[mh]);
+    const float beta = 2.f / (1.f + expf(-pb[mh]));  // as delta_heads.hip
     float kh = 0.f;
 #pragma unroll
     for (int i = 0; i < SB_DK; ++i) kh = fmaf(lane_bcast(k, i), hc[i], kh);
