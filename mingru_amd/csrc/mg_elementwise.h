@@ -265,8 +265,8 @@ struct Raw<mg_bf16, VEC> {
     for (int i = 0; i < (VEC + 1) / 2; ++i) w[i] = h << 16 | h;
   }
   // Between two uses: the compiler otherwise keeps the first use's fp32 values alive
-  // for the second instead of the packed words (228 registers against 128 in the
-  // linear forward: one workgroup per CU instead of two).
+  // for the second instead of the packed words (228 registers against 156 in the
+  // linear forward).
   __device__ __forceinline__ void repack() {
 #pragma unroll
     for (int i = 0; i < (VEC + 1) / 2; ++i) asm("" : "+v"(w[i]));

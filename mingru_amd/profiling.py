@@ -36,20 +36,23 @@ import os
 import re
 import statistics
 
+_GATE = r"kernel<(?:float, )?\d+, \d+, \d+, "
+
 # workload -> [(entry point, kernel-name pattern)], matched against the demangled
 # name with its argument list removed.
 ENTRIES = {
     "C2": [("mg_linear_scan_fwd", r"\bew_fwd_kernel<"),
            ("mg_linear_scan_bwd", r"\blinear_bwd_kernel<")],
-    # gate kernels: <columns per lane, steps per wave, waves, gate kind, decay[, launch form]>
-    "C2g": [("mg_signed_gate_scan_fwd", r"\bgate_fwd_kernel<\d+, \d+, \d+, [01], false(, \d)?>"),
-            ("mg_signed_gate_scan_bwd", r"\bgate_bwd_kernel<\d+, \d+, \d+, [01], false(, \d)?>")],
+    # gate kernels: <[element type,] columns per lane, steps per wave, waves, gate kind,
+    # decay[, launch form]>
+    "C2g": [("mg_signed_gate_scan_fwd", r"\bgate_fwd_" + _GATE + r"[01], false(, \d)?>"),
+            ("mg_signed_gate_scan_bwd", r"\bgate_bwd_" + _GATE + r"[01], false(, \d)?>")],
     "C2gd": [("mg_signed_gate_scan_decay_fwd",
-              r"\bgate_fwd_kernel<\d+, \d+, \d+, [01], true(, \d)?>"),
+              r"\bgate_fwd_" + _GATE + r"[01], true(, \d)?>"),
              ("mg_signed_gate_scan_decay_bwd",
-              r"\bgate_bwd_kernel<\d+, \d+, \d+, [01], true(, \d)?>")],
-    "C1g": [("mg_mingru_gate_scan_fwd", r"\bgate_fwd_kernel<\d+, \d+, \d+, 2, false(, \d)?>"),
-            ("mg_mingru_gate_scan_bwd", r"\bgate_bwd_kernel<\d+, \d+, \d+, 2, false(, \d)?>")],
+              r"\bgate_bwd_" + _GATE + r"[01], true(, \d)?>")],
+    "C1g": [("mg_mingru_gate_scan_fwd", r"\bgate_fwd_" + _GATE + r"2, false(, \d)?>"),
+            ("mg_mingru_gate_scan_bwd", r"\bgate_bwd_" + _GATE + r"2, false(, \d)?>")],
     "C1": [("mg_log_scan_fwd", r"\blog_fwd_kernel<"), ("mg_log_scan_bwd", r"\blog_bwd_kernel<")],
     "C3": [("mg_affine_scan_fwd", r"\baffine_fwd_kernel<2, 1,"),
            ("mg_affine_scan_bwd", r"\baffine_bwd_kernel<2, 1,")],
