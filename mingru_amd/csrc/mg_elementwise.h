@@ -30,6 +30,7 @@
 
 #include "mg_common.h"
 #include "mg_gates.h"
+#include "mg_rows.h"
 
 #include <initializer_list>
 #include <atomic>
@@ -664,14 +665,7 @@ struct EwThread {
   bool col_ok;
   unsigned cl;   // the columns the lane loads: its own, or the row's last where it has none
   int64_t b0;    // first row of the batch row, batch * T
-  // The row to load for step t: t, or the last one past the sequence end.  Loads are
-  // issued unconditionally -- a load under a condition became a branch of its own, with
-  // a wait for the register it replaced -- and a step past the end is made neutral where
-  // its value matters.  (linear_scan forward at (16, 4096, 1024) 184 -> 176 us, the
-  // MinGRU gates 186 -> 142 us, the signed gates 195 -> 182 us.)
-  __device__ __forceinline__ int64_t row(int64_t t, int64_t T) const {
-    return b0 + (t < T ? t : T - 1);
-  }
+  __device__ __forceinline__ int64_t row(int64_t t, int64_t T) const { return ew_row(b0, t, T); }
 };
 
 // The thread's chunk, lane group and columns for ticket `ticket` of the launch:
@@ -697,20 +691,6 @@ __device__ __forceinline__ EwThread ew_thread_at(const EwGeom& g, unsigned ticke
   th.b0 = (int64_t)th.bb * g.T;
   return th;
 }
-
-// Element offsets of the rows a wave loads, th.row(t0), th.row(t0 + 1), ..., times ld:
-// one scalar add a row instead of a 64-bit product.
-struct EwRows {
-  int64_t off, ld, left;
-  __device__ __forceinline__ EwRows(const EwThread& th, int64_t t0, int64_t T, int64_t ld_)
-      : off(th.row(t0, T) * ld_), ld(ld_), left(T - 1 - t0) {}
-  __device__ __forceinline__ int64_t next() {
-    const int64_t o = off;
-    off += left > 0 ? ld : 0;
-    --left;
-    return o;
-  }
-};
 
 // Runs body(ticket, epoch) for the chunks of this workgroup: with the look-back
 // (PH = EW_LOOKBACK) a persistent workgroup takes tickets until they run out
@@ -794,7 +774,7 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void ew_fwd_kernel(
   auto load = [&](unsigned ticket, Row& av, Row& bv) {
     const EwThread th = ew_thread_at<VEC, false>(g, ticket, 0u);
     const int64_t t0 = (int64_t)th.c * (WAVES * TSUB) + th.w * TSUB;
-    EwRows rows(th, t0, T, D);
+    EwRows rows(th.b0, t0, T, D);
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
       const int64_t off = rows.next();
@@ -892,13 +872,13 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void linear_bwd_kernel(
     // bp[s] = Bc_{t0+s-1} (zero before the sequence start).
     float av[TSUB][VEC], bp[TSUB][VEC], xa[TSUB][VEC], xb[TSUB][VEC];
     float Ap[VEC];
-    EwRows rows(th, t0, T, D);
+    EwRows rows(th.b0, t0, T, D);
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
       const int64_t off = rows.next();
       load_vec<VEC, NT>(av[s], a + off + th.cl);
       if constexpr (PH != EW_REDUCE)
-        load_vec<VEC>(bp[s], Bc + (t0 + s > 0 ? off - D : off) + th.cl);
+        load_vec<VEC>(bp[s], Bc + rows.before(off) + th.cl);
       load_vec<VEC, NT>(xa[s], gA + off + th.cl);
       load_vec<VEC, NT>(xb[s], gB + off + th.cl);
     }
@@ -986,7 +966,7 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void linear_bwd_bf16_kernel(
     const int64_t T = g.T, D = g.D;
 
     Raw<mg_bf16, VEC> av[TSUB], bv[TSUB], ga[TSUB], gb[TSUB];
-    EwRows rows(th, t0, T, D);
+    EwRows rows(th.b0, t0, T, D);
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
       const int64_t off = rows.next();
@@ -1105,7 +1085,7 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void log_fwd_kernel(
     // Every raw load first, then the exponentials: with each step's exponentials
     // next to its loads the compiler waited for them step by step.
     float ra[TSUB][VEC], rb[TSUB][VEC];
-    EwRows rows(th, t0, T, D);
+    EwRows rows(th.b0, t0, T, D);
     const int64_t to_lv = (int64_t)(th.bb + 1) * D;  // lv has a row more per batch row
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
@@ -1189,7 +1169,7 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void log_bwd_kernel(
 
     // a as Xf; lv and gh raw until needed.
     float ra[TSUB][VEC], lvr[TSUB][VEC], gr[TSUB][VEC];
-    EwRows rows(th, t0, T, D);
+    EwRows rows(th.b0, t0, T, D);
     const int64_t to_lv = (int64_t)(th.bb + 1) * D;  // lv has a row more per batch row
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
@@ -1394,7 +1374,7 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void gate_fwd_kernel(
   auto load = [&](unsigned ticket, Rows& r) {
     const EwThread th = ew_thread_at<VEC, false>(g, ticket, 0u);
     const int64_t t0 = (int64_t)th.c * (WAVES * TSUB) + th.w * TSUB;
-    EwRows rows(th, t0, T, g.ld);
+    EwRows rows(th.b0, t0, T, g.ld);
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
       const int64_t off = rows.next();
@@ -1497,7 +1477,7 @@ __global__ __launch_bounds__(MG_WAVE* WAVES) void gate_bwd_kernel(
   auto load = [&](unsigned ticket, Rows& r) {
     const EwThread th = ew_thread_at<VEC, true>(g, ticket, 0u);
     const int64_t t0 = (int64_t)th.c * (WAVES * TSUB) + th.w * TSUB;
-    EwRows rows(th, t0, T, g.ld), grows(th, t0, T, D);
+    EwRows rows(th.b0, t0, T, g.ld), grows(th.b0, t0, T, D);
 #pragma unroll
     for (int s = 0; s < TSUB; ++s) {
       const int64_t off = rows.next();

@@ -134,6 +134,21 @@ def test_linear_scan_long_sequence_exact(cuda):
     assert torch.equal(a.grad, (y * prev).float())
 
 
+@pytest.mark.parametrize("form", ["", "two"])
+@pytest.mark.parametrize("shape", [(1, 1, 64), (3, 1, 2048), (2, 1, 771), (300, 1, 1024),
+                                   (4096, 1, 1024)])
+def test_linear_scan_one_step(cuda, shape, form, monkeypatch):
+    """T = 1: every other step of a chunk lies past the end.  A = a, Bc = b, da = gA and
+    db = gB bit for bit; one-launch aggregate, two-launch and (from 32 MB of gradients on)
+    look-back forms, 1, 2 and 4 columns per lane."""
+    monkeypatch.setenv("MINGRU_HIP_EW_FORM", form)
+    print(f"[gpu] linear_scan one step {shape} form={form!r}", flush=True)
+    g = torch.Generator().manual_seed(5)
+    a, b, gA, gB = (torch.randn(*shape, generator=g) for _ in range(4))
+    for got, want in zip(_run_linear(a, b, gA, gB, cuda), (a, b, gA, gB)):
+        assert torch.equal(got.detach().cpu(), want)
+
+
 def _run_log(lc, lv, gh, cuda):
     lcg = lc.to(cuda).requires_grad_(True)
     lvg = lv.to(cuda).requires_grad_(True)
