@@ -31,6 +31,7 @@
 #include "mg_common.h"
 #include "mg_gates.h"
 #include "mg_rows.h"
+#include "mg_two_buffers.h"
 
 #include <initializer_list>
 #include <atomic>
@@ -713,39 +714,34 @@ __device__ __forceinline__ void ew_chunks(const EwGeom& g, unsigned* header, Bod
 // CU's single workgroup loaded, scanned and stored in turn: the signed gates on bf16
 // (16, 4096, 1024) took 196 us forward and 337 backward, as long as on fp32 at twice
 // the bytes; with two, and the loads of a chunk free of branches, 126 and 234 us.
-template <typename Rows, typename Load, typename Finish>
-__device__ __forceinline__ void ew_persistent2(const EwGeom& g, unsigned* header, Load&& load,
-                                               Finish&& finish) {
-  __shared__ unsigned s_ticket, s_epoch;
-  const unsigned chunks = (unsigned)g.n_lg * (unsigned)g.n_chunks;
-  if (threadIdx.x == 0) {
+struct EwTickets {
+  unsigned* header;
+  unsigned chunks;
+  unsigned &s_ticket, &s_epoch;  // in LDS
+  __device__ __forceinline__ void first() {
+    if (threadIdx.x != 0) return;
     const unsigned e0 =
         __hip_atomic_load(header + MG_H_EPOCH, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
     s_ticket = mg_next_ticket(header, e0, chunks);
     s_epoch = e0;
   }
-  __syncthreads();
-  unsigned t = mg_uniform(s_ticket);
-  const unsigned e = mg_uniform(s_epoch);
-  Rows r0, r1;
-  if (t < chunks) load(t, r0);
-  auto step = [&](unsigned tk, Rows& r, Rows& nr) {
-    unsigned next = 0u;
-    if (threadIdx.x == 0) next = mg_next_ticket(header, e, chunks);
-    unsigned tn = 0u;
-    finish(tk, e, r, [&] {
-      if (threadIdx.x == 0) s_ticket = next;
-      __syncthreads();
-      tn = mg_uniform(s_ticket);
-      if (tn < chunks) load(tn, nr);
-    });
-    return tn;
-  };
-  while (t < chunks) {
-    t = step(t, r0, r1);
-    if (t >= chunks) break;
-    t = step(t, r1, r0);
+  __device__ __forceinline__ unsigned next(unsigned e) {
+    return threadIdx.x == 0 ? mg_next_ticket(header, e, chunks) : 0u;
   }
+  __device__ __forceinline__ void share(unsigned t) {
+    if (threadIdx.x == 0) s_ticket = t;
+  }
+  __device__ __forceinline__ unsigned ticket() { return mg_uniform(s_ticket); }
+  __device__ __forceinline__ unsigned epoch() { return mg_uniform(s_epoch); }
+  __device__ __forceinline__ void barrier() { __syncthreads(); }
+};
+
+template <typename Rows, typename Load, typename Finish>
+__device__ __forceinline__ void ew_persistent2(const EwGeom& g, unsigned* header, Load&& load,
+                                               Finish&& finish) {
+  __shared__ unsigned s_ticket, s_epoch;
+  EwTickets wg{header, (unsigned)g.n_lg * (unsigned)g.n_chunks, s_ticket, s_epoch};
+  ew_two_buffers<Rows>(wg, wg.chunks, load, finish);
 }
 
 // ---------------------------------------------------------------------------

@@ -28,3 +28,9 @@ def test_scan_rows_stay_in_the_tensors(tmp_path):
     """Every row the elementwise scans load, steps past the end included, for sequences of
     one step and more."""
     _run("host_rows", tmp_path)
+
+
+def test_two_buffer_waves_take_the_same_tickets(tmp_path):
+    """The persistent form with two row buffers: a wave that reads the shared ticket late
+    still takes the workgroup's chunk and not the next one."""
+    _run("host_two_buffers", tmp_path)
