@@ -361,7 +361,7 @@ def _join_backend(x: torch.Tensor, linears, impl: str):
     if torch.nn.modules.module._has_any_global_hook():
         return None
     if linears[0].weight.dtype not in (torch.float32, torch.bfloat16) or (
-        torch.is_autocast_enabled() and torch.get_autocast_gpu_dtype() != torch.bfloat16
+        torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") != torch.bfloat16
     ):
         return None
     like = None
@@ -1583,7 +1583,10 @@ class DeltaMinGRU(DecayMixin, nn.Module):
     def _joined_forward(self, x, H, log_gamma=None):
         """The delta kernels on heads formed from one joined projection, or ``None``
         (silent in every mode) for the separate projections and their seam, which apply
-        the mode's rules."""
+        the mode's rules.  Under autocast the separate form normalises the keys in fp32 and
+        scans in fp32, which one joined product in the autocast type would not."""
+        if torch.is_autocast_enabled():
+            return None
         linears = (self.linear_q, *self.linear_k, *self.linear_v, *self.linear_beta)
         backend = _join_backend(x, linears, "delta_heads_impl")
         if backend is None or max(self.d_k, self.d_v) > _DELTA_AUTO_MAX_DK:

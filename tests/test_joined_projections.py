@@ -95,6 +95,49 @@ def test_other_projections_stay_separate(monkeypatch, why):
         assert seen == [1]
 
 
+def _fake_delta(monkeypatch, calls):
+    """The fake backend with the delta entry points; the scan keeps the true envelope."""
+    _fake(monkeypatch, calls)
+    fake = sys.modules[BACKEND]
+
+    def heads(P, H, nh, dk, dv):
+        calls.append("heads")
+        B, T, _ = P.shape
+        return tuple(P.new_zeros(B, H, T, *s) for s in ((dk,), (nh, dk), (nh, dv), (nh,)))
+
+    def scan(Q, K, V, beta, *rest, chunk_size):
+        if K.shape[3] * chunk_size > 128:
+            raise fake.ScanFallback("nh * chunk_size")
+        calls.append("scan")
+        return V[..., 0, :], rest[-1]
+
+    fake.delta_heads_impl = heads
+    fake.delta_scan_impl = fake.delta_gated_scan_impl = scan
+    return fake
+
+
+@pytest.mark.parametrize("decay", [None, "learnable"])
+def test_delta_heads_stay_separate_under_autocast(monkeypatch, decay):
+    """Under autocast the keys are normalised in fp32 and the scan runs in fp32; one joined
+    bf16 product would round them and move the whole layer to the bf16 kernels."""
+    calls = []
+    _fake_delta(monkeypatch, calls)
+    m = DeltaMinGRU(8, 8, n_heads=2, decay=decay)
+    x, dt = torch.randn(2, 6, 8), torch.rand(2, 6) if decay else None
+    m(x, delta_t=dt)
+    assert calls == ["heads", "scan"]
+    calls.clear()
+    kind = torch.get_autocast_dtype("cuda")
+    torch.set_autocast_enabled("cuda", True)
+    torch.set_autocast_dtype("cuda", torch.bfloat16)
+    try:
+        m(x, delta_t=dt)
+    finally:
+        torch.set_autocast_dtype("cuda", kind)
+        torch.set_autocast_enabled("cuda", False)
+    assert calls == ["scan"]
+
+
 def _pair(cuda, m, dtype):
     joined = m.to(cuda, dtype)
     separate = copy.deepcopy(joined)
@@ -174,3 +217,38 @@ def test_joined_equals_separate(cuda, case, dtype, monkeypatch):
         assert a.dtype == b.dtype and a.shape == b.shape
         assert _off(a, r) <= 1.5 * _off(b, r) + 2.0**-8, (
             f"output {i}: joined {_off(a, r):.2e}, separate {_off(b, r):.2e} off float64")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", range(len(MODULES + GIVENS)))
+def test_joined_equals_separate_under_autocast(cuda, case, monkeypatch):
+    """fp32 modules under bf16 autocast: the joined gates round where the separate ones do
+    (their products' outputs), and the delta and Givens layers, whose separate forms compute
+    their heads in fp32, don't join at all: their outputs are the same to the last bit."""
+    gates = case < 6
+    build, B, T, decay = (MODULES + GIVENS)[case]
+    print(f"[gpu] joined projections under autocast case={case}", flush=True)
+    monkeypatch.setenv("MINGRU_SCAN", "hip")
+    torch.manual_seed(100 + case)
+    joined, separate = _pair(cuda, build(), torch.float32)
+    x = torch.randn(B, T, joined.input_size, device=cuda)
+    dt = torch.rand(B, T, device=cuda) if decay else None
+    res = []
+    for m in (joined, separate):
+        xi = x.clone().requires_grad_()
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = m(xi, delta_t=dt) if decay else m(xi)
+        gy = torch.randn(y.shape, generator=torch.Generator().manual_seed(9)).to(cuda, y.dtype)
+        res.append([y.detach(), *torch.autograd.grad(y, [xi, *m.parameters()], gy)])
+    monkeypatch.setenv("MINGRU_SCAN", "eager")
+    ref = copy.deepcopy(joined).double()
+    xi = x.double().requires_grad_()
+    y = ref(xi, delta_t=dt.double()) if decay else ref(xi)
+    exact = [y.detach(), *torch.autograd.grad(y, [xi, *ref.parameters()], gy.double())]
+    for i, (a, b, r) in enumerate(zip(*res, exact)):
+        assert a.dtype == b.dtype and a.shape == b.shape
+        if gates:
+            assert _off(a, r) <= 1.5 * _off(b, r) + 2.0**-8, (
+                f"output {i}: joined {_off(a, r):.2e}, separate {_off(b, r):.2e} off float64")
+        else:
+            assert torch.equal(a, b), f"output {i}"
