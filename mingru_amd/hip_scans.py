@@ -1781,17 +1781,29 @@ _BLOCK_STEP_GROUP = 16
 _BLOCK_STEP_MAX_LDS = 64 << 10
 
 
-def _step_project(x, ln, linears, epi: int, res, out, dtype: int) -> None:
+def _step_project(x, ln, linears, rows, epi: int, res, out, dtype: int) -> None:
     n = len(linears)
-    K = x.shape[1]
+    B, K = x.shape
     pointers = ctypes.c_void_p * n
     w = pointers(*[p[0].data_ptr() for p in linears])
     b = pointers(*[None if p[1] is None else p[1].data_ptr() for p in linears])
-    rows = (ctypes.c_int * n)(*[p[0].shape[0] for p in linears])
     lw, lb, eps = (None, None, 0.0) if ln is None else ln
-    _call("mg_step_project", dtype, _ptr(x), int(x.dtype == torch.float32), x.shape[0], K,
-          _ptr(lw), _ptr(lb), eps, n, w, b, rows, epi, _ptr(res), _ptr(out),
+    _call("mg_step_project", dtype, _ptr(x), int(x.dtype == torch.float32), B, K,
+          _ptr(lw), _ptr(lb), eps, n, w, b, (ctypes.c_int * n)(*rows), epi, _ptr(res), _ptr(out),
           int(out.dtype == torch.float32), _stream(x))
+
+
+def _projection_rows(pairs, K: int) -> list:
+    """The row counts of projections (weight, bias) of ``K`` columns."""
+    rows = []
+    for w, b in pairs:
+        shape = w.shape
+        if len(shape) != 2 or shape[1] != K or (b is not None and b.shape != (shape[0],)):
+            raise ScanFallback(
+                f"block step: a projection's shape {tuple(shape)}, bias "
+                f"{None if b is None else tuple(b.shape)}, on rows of {K}")
+        rows.append(shape[0])
+    return rows
 
 
 def block_step_impl(kind: str, x, ln1, proj, h_prev, gamma, delta, ln2, mlp):
@@ -1810,27 +1822,47 @@ def block_step_impl(kind: str, x, ln1, proj, h_prev, gamma, delta, ln2, mlp):
         raise ScanFallback(f"block step: {x.dtype} x {tuple(x.shape)}")
     if d % 4 or B * d > _BLOCK_STEP_MAX_ELEMENTS or 4 * min(B, _BLOCK_STEP_GROUP) * d > _BLOCK_STEP_MAX_LDS:
         raise ScanFallback(f"block step: width {d} at {B} sequences")
-    pairs = [*proj, *(mlp or ()), *([delta[4]] if delta else ())]
-    ts = [x, h_prev, *ln1[:2], *(t for p in pairs for t in p if t is not None)]
+    # Every shape the kernels take for granted: they read K elements of each row, and the
+    # layers of an edited block may not fit together.
+    rows, pairs, row, lns = _projection_rows(proj, d), [*proj], (d,), [*ln1[:2]]
+    if delta:
+        H, nh, dk, dv, out_proj = delta
+        width, inner = H * dk * dv, H * dv
+        fits = (rows == [H * dk] * (1 + nh) + [H * dv] * nh + [H] * nh
+                and _projection_rows([out_proj], inner) == [d])
+        pairs.append(out_proj)
+    else:
+        width, inner = d, d
+        fits = rows == [d] * (2 if kind == "mingru" else 3)
+    up = None
     if mlp:
-        ts += ln2[:2]
-    dev = x.device
-    for t in ts:
-        if t.dtype != x.dtype or t.device != dev or not t.is_contiguous() or t.data_ptr() % 16:
-            raise ScanFallback("block step needs dense, aligned tensors of one type and device")
-    if dev.type != "cuda" or any(p[0].shape[1] % 4 for p in pairs):
+        up = _projection_rows(mlp[:1], d)
+        fits = fits and _projection_rows(mlp[1:], up[0]) == [d]
+        pairs += mlp
+        lns += ln2[:2]
+    for t in lns:
+        fits = fits and t.shape == row
+    if gamma is not None:
+        fits = fits and gamma.shape == (B, H if delta else d) and gamma.device == x.device
+    if not fits or h_prev.shape != (B, width):
+        raise ScanFallback(f"block step: shapes of the parts disagree at width {d}")
+    if not x.is_cuda or inner % 4 or (mlp and up[0] % 4):
         raise ScanFallback("block step: GPU tensors with rows of whole 4-element pieces")
-    tag = 1 if x.dtype == torch.bfloat16 else 0
+    dev, dtype, index = x.device, x.dtype, x.get_device()
+    for t in (x, h_prev, *lns, *(t for p in pairs for t in p if t is not None)):
+        if (t.dtype != dtype or t.get_device() != index or not t.is_contiguous()
+                or t.data_ptr() % 16):
+            raise ScanFallback("block step needs dense, aligned tensors of one type and device")
+    tag = 1 if dtype == torch.bfloat16 else 0
     mid = torch.empty_like(x)  # x + the mixer's output
     state = torch.empty_like(h_prev)
     if kind == "delta":
-        H, nh, dk, dv, out_proj = delta
         P = torch.empty(B, H * (dk + nh * (dk + dv) + nh), dtype=torch.float32, device=dev)
-        _step_project(x, ln1, proj, 0, None, P, tag)
+        _step_project(x, ln1, proj, rows, 0, None, P, tag)
         y = torch.empty(B, H * dv, dtype=torch.float32, device=dev)
         _call("mg_delta_step_heads", tag, _ptr(h_prev), _ptr(P), _ptr(gamma), _ptr(state),
               _ptr(y), B, H, nh, dk, dv, _stream(x))
-        _step_project(y, None, [out_proj], 2, x, mid, tag)
+        _step_project(y, None, [out_proj], [d], 2, x, mid, tag)
     else:
         (w0, b0), (w1, b1) = proj[:2]
         w2, b2 = proj[2] if len(proj) == 3 else (None, None)
@@ -1839,10 +1871,10 @@ def block_step_impl(kind: str, x, ln1, proj, h_prev, gamma, delta, ln2, mlp):
               _ptr(gamma), _ptr(h_prev), _ptr(state), _ptr(mid), d, _stream(x))
     if not mlp:
         return mid, state
-    hidden = torch.empty(B, mlp[0][0].shape[0], dtype=torch.float32, device=dev)
-    _step_project(mid, ln2, mlp[:1], 1, None, hidden, tag)
+    hidden = torch.empty(B, up[0], dtype=torch.float32, device=dev)
+    _step_project(mid, ln2, mlp[:1], up, 1, None, hidden, tag)
     out = torch.empty_like(x)
-    _step_project(hidden, None, mlp[1:], 2, mid, out, tag)
+    _step_project(hidden, None, mlp[1:], [d], 2, mid, out, tag)
     return out, state
 
 

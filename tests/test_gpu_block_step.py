@@ -99,6 +99,20 @@ def test_block_step_declines(cuda, monkeypatch):
     torch.testing.assert_close(y, m.step(wide[:, ::2].contiguous(), None)[0], rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("mode", ["auto", "hip"])
+def test_block_step_of_layers_that_do_not_fit(cuda, mode, monkeypatch):
+    """An edited block whose layers disagree raises torch's error, as its forward does."""
+    monkeypatch.setenv("MINGRU_SCAN", mode)
+    m = MinGRUBlock(64, 2).to(cuda).eval()
+    m.mlp[0] = torch.nn.Linear(64, 256).to(cuda)  # wider than mlp[3] reads
+    x = torch.randn(2, 64, device=cuda)
+    with pytest.raises(RuntimeError, match="shapes cannot be multiplied"):
+        m.step(x, None)
+    m.mlp[3] = torch.nn.Linear(256, 64).to(cuda)
+    y, _ = m.step(x, None)
+    torch.testing.assert_close(y, m(x[:, None])[0][:, 0], rtol=1e-5, atol=1e-5)
+
+
 def test_stack_stream_equals_forward(cuda, monkeypatch):
     """A streamed hybrid stack equals its forward over the sequence."""
     monkeypatch.setenv("MINGRU_SCAN", "hip")
