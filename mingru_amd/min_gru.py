@@ -345,15 +345,15 @@ def _is_plain(m: nn.Module, cls: type) -> bool:
     )
 
 
-def _join_backend(x: torch.Tensor, linears, impl: str):
+def _join_backend(x: torch.Tensor, linears, widths, impl: str):
     """The backend, if it has ``impl`` and one joined projection of ``x`` may stand in for
-    ``linears``; else ``None``.
+    ``linears`` of ``widths`` outputs; else ``None``.
 
     Joined, the projections are one matrix product each way instead of one per layer, and
     the input's gradient needs no sum (fwd+bwd of three 1024-wide bf16 projections of 16384
     rows: 614 -> 360 us).  Only for what calling each layer would compute anyway: plain
-    ``nn.Linear`` modules without hooks, alike in dtype, device, bias and whether they are
-    trained.
+    ``nn.Linear`` modules without hooks, of the widths that the joined rows are split at,
+    alike in dtype, device, bias and whether they are trained.
     """
     rows = x.numel() // max(1, x.shape[-1])
     if not torch.is_grad_enabled() and rows < _JOIN_MIN_ROWS:
@@ -364,11 +364,15 @@ def _join_backend(x: torch.Tensor, linears, impl: str):
         torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") != torch.bfloat16
     ):
         return None
-    like = None
-    for m in linears:
+    if len(linears) != len(widths):
+        return None
+    like, columns = None, x.shape[-1]
+    for m, width in zip(linears, widths):
         if not _is_plain(m, nn.Linear):
             return None
         w, b = m.weight, m.bias
+        if w.shape != (width, columns) or (b is not None and b.shape != (width,)):
+            return None
         this = (w.dtype, w.device, w.requires_grad,
                 None if b is None else (b.dtype, b.device, b.requires_grad))
         if like is not None and this != like:
@@ -389,8 +393,10 @@ def _join_linears(x: torch.Tensor, linears) -> torch.Tensor:
     return F.linear(x, torch.cat([m.weight for m in linears]), bias)
 
 
-def _dispatch_joined_gate_scan(kind: str, x, linears, h0, dt=None, lam=None, h0_const=0.0):
-    """The fused gate scan from one joined projection of ``x``, or ``None``.
+def _dispatch_joined_gate_scan(kind: str, x, linears, width, h0, dt=None, lam=None,
+                               h0_const=0.0):
+    """The fused gate scan from one joined projection of ``x`` (``width`` columns per layer),
+    or ``None``.
 
     ``None`` (silent in every mode) leads to the separate projections and
     ``_dispatch_signed_gate_scan`` / ``_dispatch_mingru_gate_scan``, which apply the
@@ -398,7 +404,7 @@ def _dispatch_joined_gate_scan(kind: str, x, linears, h0, dt=None, lam=None, h0_
     """
     if _resolve_scan_mode(x.is_cuda) is None or x.dim() != 3 or x.numel() == 0:
         return None
-    backend = _join_backend(x, linears, "gate_scan_packed_impl")
+    backend = _join_backend(x, linears, (width,) * len(linears), "gate_scan_packed_impl")
     if backend is None:
         return None
     try:
@@ -965,7 +971,8 @@ class MinGRU(DecayMixin, nn.Module):
             )
             log_h_0 = h_0.clamp_min(torch.finfo(h_0.dtype).tiny).log()
         dt = self._prepare_decay(delta_t, canonical_ndim=2)
-        h = _dispatch_joined_gate_scan("mingru", x, (self.linear_z, self.linear_h), log_h_0, dt,
+        h = _dispatch_joined_gate_scan("mingru", x, (self.linear_z, self.linear_h),
+                                       self.hidden_size, log_h_0, dt,
                                        None if dt is None else self._decay_lambda(),
                                        h0_const=math.log(0.5))
         if h is not None:
@@ -1059,7 +1066,8 @@ class SignedMinGRU(DecayMixin, nn.Module):
             h_0 = self.h0.expand(x.size(0), 1, self.hidden_size)
         dt = self._prepare_decay(delta_t, canonical_ndim=2)
         h = _dispatch_joined_gate_scan("signed_coupled" if self.coupled else "signed", x,
-                                       (self.linear_s, self.linear_z, self.linear_h), h_0, dt,
+                                       (self.linear_s, self.linear_z, self.linear_h),
+                                       self.hidden_size, h_0, dt,
                                        None if dt is None else self._decay_lambda())
         if h is not None:
             return h
@@ -1372,7 +1380,8 @@ class GivensMinGRU(DecayMixin, nn.Module):
         if (self.k != 8 or x.dim() != 3 or x.numel() == 0 or torch.is_autocast_enabled()
                 or self.linear_z.weight.dtype != torch.float32):
             return None
-        backend = _join_backend(x, linears, "angle_joined_scan_impl")
+        widths = (self.hidden_size, self.hidden_size, self.n_blocks * self.rounds * 4)
+        backend = _join_backend(x, linears, widths, "angle_joined_scan_impl")
         if backend is None:
             return None
         B, T, _ = x.shape
@@ -1588,7 +1597,9 @@ class DeltaMinGRU(DecayMixin, nn.Module):
         if torch.is_autocast_enabled():
             return None
         linears = (self.linear_q, *self.linear_k, *self.linear_v, *self.linear_beta)
-        backend = _join_backend(x, linears, "delta_heads_impl")
+        H_k, H_v, nh = self.n_heads * self.d_k, self.n_heads * self.d_v, self.nh
+        widths = [H_k] * (1 + nh) + [H_v] * nh + [self.n_heads] * nh
+        backend = _join_backend(x, linears, widths, "delta_heads_impl")
         if backend is None or max(self.d_k, self.d_v) > _DELTA_AUTO_MAX_DK:
             return None
         try:

@@ -138,6 +138,54 @@ def test_delta_heads_stay_separate_under_autocast(monkeypatch, decay):
     assert calls == ["scan"]
 
 
+WIDTHS = {
+    # Layers edited to widths that add up to the right sum, or to a multiple of it.
+    "mingru": (lambda: MinGRU(4, 6), {"linear_z": (4, 8), "linear_h": (4, 4)}),
+    "mingru wider": (lambda: MinGRU(4, 6), {"linear_h": (4, 10)}),
+    "signed": (lambda: SignedMinGRU(4, 6), {"linear_s": (4, 5), "linear_h": (4, 7)}),
+    "givens": (lambda: GivensMinGRU(4, 16), {"linear_z": (4, 12), "linear_h": (4, 20)}),
+    "delta": (lambda: DeltaMinGRU(8, 8, n_heads=2), {"linear_q": (8, 6), "linear_k.0": (8, 10)}),
+    "delta beta": (lambda: DeltaMinGRU(8, 8, n_heads=2), {"linear_v.0": (8, 9),
+                                                          "linear_beta.0": (8, 1)}),
+    "delta lists": (lambda: DeltaMinGRU(8, 8, n_heads=2), {"linear_k.1": (8, 8),
+                                                           "linear_v.1": (8, 8)}),
+}
+
+
+@pytest.mark.parametrize("case", WIDTHS)
+def test_projections_of_other_widths_stay_separate(monkeypatch, case):
+    """Side by side, rows of another split would pass for the right ones; one by one, torch
+    refuses them."""
+    calls = []
+    fake = _fake_delta(monkeypatch, calls)
+    fake.angle_joined_scan_impl = lambda *a: calls.append("joined")
+    build, widths = WIDTHS[case]
+    m = build()
+    for name, (i, o) in widths.items():
+        parent, _, leaf = name.rpartition(".")
+        m.get_submodule(parent).add_module(leaf, nn.Linear(i, o))
+    monkeypatch.setattr(mg, "_join_linears", lambda *a: calls.append("product") or _real(*a))
+    try:
+        m(torch.randn(2, 5, m.input_size))
+    except (RuntimeError, IndexError):
+        pass
+    assert "product" not in calls, calls
+
+
+_real = mg._join_linears
+
+
+def test_a_bias_that_broadcasts_stays_separate(monkeypatch):
+    calls = []
+    _fake(monkeypatch, calls)
+    m = MinGRU(4, 6)
+    m.linear_z.bias = nn.Parameter(torch.zeros(1))
+    m.linear_h.bias = nn.Parameter(torch.zeros(11))
+    with pytest.raises(RuntimeError, match="size"):
+        m(torch.randn(2, 5, 4))
+    assert calls == []
+
+
 def _pair(cuda, m, dtype):
     joined = m.to(cuda, dtype)
     separate = copy.deepcopy(joined)
