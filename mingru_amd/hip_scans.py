@@ -42,7 +42,9 @@ __all__ = [
     "gate_step_impl",
     "delta_step_impl",
     "angle_joined_scan_impl",
+    "angle_joined_reason",
     "delta_heads_impl",
+    "delta_joined_reason",
     "block_step_impl",
     "workspace_errors",
     "LookbackError",
@@ -1388,6 +1390,16 @@ class _JoinedAngleGatedFn(torch.autograd.Function):
         return dP, None if dgm is None else dgm.to(gdt), dh0.to(h0dt), None
 
 
+def angle_joined_reason(rounds: int, h0_dtype) -> str | None:
+    """Why ``angle_joined_scan_impl`` would decline a joined projection of ``rounds`` rounds
+    and this initial state, asked before the product; ``None`` where it would not."""
+    if not 1 <= rounds <= _ANGLE_MAX_ROT:
+        return f"joined angle scan needs 1 to {_ANGLE_MAX_ROT} rounds (got {rounds})"
+    if h0_dtype == torch.float64 or not h0_dtype.is_floating_point:
+        return f"joined angle scan computes in fp32 (got an initial state of {h0_dtype})"
+    return None
+
+
 def angle_joined_scan_impl(P, gamma, h0, rounds: int):
     """``angle_gated_scan_impl`` for GivensMinGRU's 8x8 brick-wall blocks on one joined
     fp32 projection: ``P`` (B, T, n (16 + 4 rounds)), its rows ``z | hpre | theta``;
@@ -1583,6 +1595,17 @@ class _DeltaHeadsFn(torch.autograd.Function):
         _call("mg_delta_heads_bwd", _ptr(K), _ptr(beta), _ptr(nrm), *(_ptr(t) for t in grads),
               _ptr(dP), *ctx.dims, _stream(K))
         return dP, None, None, None, None
+
+
+def delta_joined_reason(*, is_cuda: bool, dtype, h0_dtype, d_k: int, d_v: int, nh: int,
+                        chunk_size: int) -> str | None:
+    """Why ``delta_heads_impl`` or the scan after it would decline heads of ``dtype`` from
+    one joined projection, asked before the product; ``None`` where neither would."""
+    if dtype not in (torch.float32, torch.bfloat16):
+        return f"joined delta heads need fp32 or bf16 (got {dtype})"
+    return _delta_envelope_reason(is_cuda=is_cuda, q_dtype=dtype, k_dtype=dtype, v_dtype=dtype,
+                                  beta_dtype=dtype, h0_dtype=h0_dtype, d_k=d_k, d_v=d_v,
+                                  chunk_size=chunk_size, nh=nh)
 
 
 def delta_heads_impl(P: torch.Tensor, n_heads: int, nh: int, d_k: int, d_v: int):

@@ -404,6 +404,13 @@ def _dispatch_joined_gate_scan(kind: str, x, linears, width, h0, dt=None, lam=No
     """
     if _resolve_scan_mode(x.is_cuda) is None or x.dim() != 3 or x.numel() == 0:
         return None
+    # What the kernel would decline whatever the projection holds, before the product.
+    B, T, _ = x.shape
+    if h0 is not None and (h0.shape != (B, 1, width) or h0.device != x.device
+                           or h0.dtype == torch.float64 or not h0.dtype.is_floating_point):
+        return None
+    if dt is not None and (dt.shape != (B, T) or dt.device != x.device):
+        return None
     backend = _join_backend(x, linears, (width,) * len(linears), "gate_scan_packed_impl")
     if backend is None:
         return None
@@ -1382,7 +1389,8 @@ class GivensMinGRU(DecayMixin, nn.Module):
             return None
         widths = (self.hidden_size, self.hidden_size, self.n_blocks * self.rounds * 4)
         backend = _join_backend(x, linears, widths, "angle_joined_scan_impl")
-        if backend is None:
+        if (backend is None or h0_blocks.device != x.device
+                or backend.angle_joined_reason(self.rounds, h0_blocks.dtype) is not None):
             return None
         B, T, _ = x.shape
         gamma = self._decay_gamma(dt).expand(B, T, self.n_blocks) if dt is not None else None
@@ -1600,7 +1608,9 @@ class DeltaMinGRU(DecayMixin, nn.Module):
         H_k, H_v, nh = self.n_heads * self.d_k, self.n_heads * self.d_v, self.nh
         widths = [H_k] * (1 + nh) + [H_v] * nh + [self.n_heads] * nh
         backend = _join_backend(x, linears, widths, "delta_heads_impl")
-        if backend is None or max(self.d_k, self.d_v) > _DELTA_AUTO_MAX_DK:
+        if backend is None or H.device != x.device or backend.delta_joined_reason(
+                is_cuda=x.is_cuda, dtype=self.linear_q.weight.dtype, h0_dtype=H.dtype,
+                d_k=self.d_k, d_v=self.d_v, nh=self.nh, chunk_size=self.chunk_size) is not None:
             return None
         try:
             heads = backend.delta_heads_impl(_join_linears(x, linears), self.n_heads, self.nh,

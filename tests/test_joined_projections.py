@@ -10,6 +10,7 @@ be no further off than the separate one, plus one rounding of the output (2^-8).
 """
 
 import copy
+import importlib
 import sys
 import types
 
@@ -22,6 +23,7 @@ from mingru_amd import DeltaMinGRU, GivensMinGRU, MinGRU, SignedMinGRU
 from mingru_amd import min_gru as mg
 
 BACKEND = "mingru_amd.hip_scans"
+HIP_SCANS = importlib.import_module(BACKEND)
 
 
 def _fake(monkeypatch, calls):
@@ -113,6 +115,10 @@ def _fake_delta(monkeypatch, calls):
 
     fake.delta_heads_impl = heads
     fake.delta_scan_impl = fake.delta_gated_scan_impl = scan
+    fake.delta_joined_reason = lambda **kw: HIP_SCANS.delta_joined_reason(
+        **dict(kw, is_cuda=True))
+    fake.angle_joined_scan_impl = lambda *a: calls.append("joined")
+    fake.angle_joined_reason = HIP_SCANS.angle_joined_reason
     return fake
 
 
@@ -157,8 +163,7 @@ def test_projections_of_other_widths_stay_separate(monkeypatch, case):
     """Side by side, rows of another split would pass for the right ones; one by one, torch
     refuses them."""
     calls = []
-    fake = _fake_delta(monkeypatch, calls)
-    fake.angle_joined_scan_impl = lambda *a: calls.append("joined")
+    _fake_delta(monkeypatch, calls)
     build, widths = WIDTHS[case]
     m = build()
     for name, (i, o) in widths.items():
@@ -173,6 +178,34 @@ def test_projections_of_other_widths_stay_separate(monkeypatch, case):
 
 
 _real = mg._join_linears
+
+
+OUTSIDE = {
+    # module, delta_t's shape, h_0: what the kernels decline whatever the projection holds.
+    "delta microsteps": (lambda: DeltaMinGRU(8, 8, n_heads=2, nh=3), None, None),
+    "delta chunk": (lambda: DeltaMinGRU(8, 8, n_heads=2, chunk_size=65, decay="fixed"), (2, 5), None),
+    "delta state": (lambda: DeltaMinGRU(8, 8, n_heads=2), None, torch.zeros(2, 1, 32).double()),
+    "h0 for every row": (lambda: SignedMinGRU(4, 6), None, torch.zeros(1, 1, 6)),
+    "h0 type": (lambda: MinGRU(4, 6), None, torch.ones(2, 1, 6).double()),
+    "one gap for every row": (lambda: SignedMinGRU(4, 6, decay="fixed"), (1, 5), None),
+    "rounds": (lambda: GivensMinGRU(4, 16, rounds=65), None, None),
+    "givens state": (lambda: GivensMinGRU(4, 16), None, torch.zeros(2, 1, 16).double()),
+}
+
+
+@pytest.mark.parametrize("case", OUTSIDE)
+def test_a_call_the_kernels_decline_projects_nothing_first(monkeypatch, case):
+    """The envelope is asked before the joined product, which would be dropped."""
+    calls = []
+    _fake_delta(monkeypatch, calls)
+    build, gaps, h0 = OUTSIDE[case]
+    monkeypatch.setattr(mg, "_join_linears", lambda *a: calls.append("product") or _real(*a))
+    m = build()
+    try:
+        m(torch.randn(2, 5, m.input_size), h0, None if gaps is None else torch.rand(*gaps))
+    except RuntimeError as exc:
+        assert "MINGRU_SCAN=hip" in str(exc)  # the separate form's seam
+    assert "product" not in calls, calls
 
 
 def test_a_bias_that_broadcasts_stays_separate(monkeypatch):
