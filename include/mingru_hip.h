@@ -331,7 +331,8 @@ int mg_delta_gated_bwd(const void* Q, const void* K, const void* V, const void* 
  * + nh), rows q (H,dk) | k (nh,H,dk) | v (nh,H,dv) | beta (nh,H), in dtype (0 fp32,
  * 1 bf16) -> Q (B,H,T,dk), K (B,H,T,nh,dk) of unit norm, V (B,H,T,nh,dv), beta (B,H,T,nh)
  * and, if not NULL, nrm (B,H,T,nh) fp32: the keys' norms (at least 1e-12, negated where
- * that bound was taken), which the backward needs.  dk, dv <= 64. */
+ * that bound was taken), which the backward needs.  dk, dv <= 64, and B T H times the lanes
+ * of a head (16, 32 or 64, the smallest that holds max(dk, dv)) at most 2^32 - 256. */
 int mg_delta_heads_fwd(const void* P, void* Q, void* K, void* V, void* beta, float* nrm, int64_t B,
                        int64_t T, int H, int nh, int dk, int dv, int dtype, mg_stream_t stream);
 /* K, beta, nrm = the forward's; dQ, dK, dV, dbeta in the kernel layouts -> dP (B,T,N). */

@@ -129,21 +129,27 @@ __global__ __launch_bounds__(HD_NT) void heads_bwd(const E* __restrict__ K,
   }
 }
 
+// Lanes of a (token, head)'s group: the smallest that holds its rows.
+int hd_group(const HdGeom& g) {
+  const int d = g.dk > g.dv ? g.dk : g.dv;
+  return d <= 16 ? 16 : d <= 32 ? 32 : 64;
+}
+
 bool hd_geom(HdGeom& g, int64_t B, int64_t T, int H, int nh, int dk, int dv, int dtype) {
   if (B <= 0 || T <= 0 || H <= 0 || nh <= 0 || dk <= 0 || dk > 64 || dv <= 0 || dv > 64 ||
       (dtype & ~1))
     return false;
   g = HdGeom{B * T * H, T, (int64_t)H * (dk + (int64_t)nh * (dk + dv) + nh), H, nh, dk, dv};
-  return g.rows < (1ll << 31);
+  return g.rows * hd_group(g) <= (1ll << 32) - HD_NT;  // a launch takes fewer than 2^32 threads
 }
 
 // f(element tag, group size) for the dtype (0 fp32, 1 bf16) and the head dims.
 template <typename F>
 int hd_pick(int dtype, const HdGeom& g, F&& f) {
-  const int d = g.dk > g.dv ? g.dk : g.dv;
+  const int group = hd_group(g);
   auto by_group = [&](auto e) {
-    if (d <= 16) f(e, std::integral_constant<int, 16>{});
-    else if (d <= 32) f(e, std::integral_constant<int, 32>{});
+    if (group == 16) f(e, std::integral_constant<int, 16>{});
+    else if (group == 32) f(e, std::integral_constant<int, 32>{});
     else f(e, std::integral_constant<int, 64>{});
   };
   if (dtype) by_group(u16{});

@@ -1597,12 +1597,17 @@ class _DeltaHeadsFn(torch.autograd.Function):
         return dP, None, None, None, None
 
 
-def delta_joined_reason(*, is_cuda: bool, dtype, h0_dtype, d_k: int, d_v: int, nh: int,
-                        chunk_size: int) -> str | None:
+def delta_joined_reason(*, is_cuda: bool, dtype, h0_dtype, tokens: int, n_heads: int, d_k: int,
+                        d_v: int, nh: int, chunk_size: int) -> str | None:
     """Why ``delta_heads_impl`` or the scan after it would decline heads of ``dtype`` from
-    one joined projection, asked before the product; ``None`` where neither would."""
+    the joined projection of ``tokens`` rows, asked before the product; ``None`` where
+    neither would."""
     if dtype not in (torch.float32, torch.bfloat16):
         return f"joined delta heads need fp32 or bf16 (got {dtype})"
+    # One launch of whole 256-thread workgroups, 16, 32 or 64 lanes for a token's head.
+    lanes = next((g for g in (16, 32) if max(d_k, d_v) <= g), 64)
+    if tokens * n_heads * lanes > 2**32 - 256:
+        return f"joined delta heads: {tokens} tokens of {n_heads} heads pass one launch"
     return _delta_envelope_reason(is_cuda=is_cuda, q_dtype=dtype, k_dtype=dtype, v_dtype=dtype,
                                   beta_dtype=dtype, h0_dtype=h0_dtype, d_k=d_k, d_v=d_v,
                                   chunk_size=chunk_size, nh=nh)

@@ -1610,7 +1610,8 @@ class DeltaMinGRU(DecayMixin, nn.Module):
         backend = _join_backend(x, linears, widths, "delta_heads_impl")
         if backend is None or H.device != x.device or backend.delta_joined_reason(
                 is_cuda=x.is_cuda, dtype=self.linear_q.weight.dtype, h0_dtype=H.dtype,
-                d_k=self.d_k, d_v=self.d_v, nh=self.nh, chunk_size=self.chunk_size) is not None:
+                tokens=x.shape[0] * x.shape[1], n_heads=self.n_heads, d_k=self.d_k,
+                d_v=self.d_v, nh=self.nh, chunk_size=self.chunk_size) is not None:
             return None
         try:
             heads = backend.delta_heads_impl(_join_linears(x, linears), self.n_heads, self.nh,

@@ -10,6 +10,7 @@ be no further off than the separate one, plus one rounding of the output (2^-8).
 """
 
 import copy
+import ctypes
 import importlib
 import sys
 import types
@@ -206,6 +207,23 @@ def test_a_call_the_kernels_decline_projects_nothing_first(monkeypatch, case):
     except RuntimeError as exc:
         assert "MINGRU_SCAN=hip" in str(exc)  # the separate form's seam
     assert "product" not in calls, calls
+
+
+@pytest.mark.parametrize("d,lanes", [(16, 16), (17, 32), (64, 64)])
+def test_delta_heads_stay_inside_one_launch(d, lanes):
+    """A launch takes fewer than 2^32 threads: past that many lanes the heads are declined
+    before the product, and the C entries refuse them (host checks: nothing is launched)."""
+    from mingru_amd import _native
+
+    kw = dict(is_cuda=True, dtype=torch.bfloat16, h0_dtype=torch.float32, d_k=d, d_v=8, nh=1,
+              chunk_size=64, n_heads=8)
+    tokens = (2**32 - 256) // (8 * lanes)  # of 8 heads
+    assert HIP_SCANS.delta_joined_reason(**kw, tokens=tokens) is None
+    assert "tokens" in HIP_SCANS.delta_joined_reason(**kw, tokens=tokens + 1)
+    lib, one = _native.load(), ctypes.c_void_p(16)
+    dims = (1, tokens + 1, 8, 1, d, 8, 1)
+    assert lib.mg_delta_heads_fwd(*[one] * 6, *dims, None) == 1
+    assert lib.mg_delta_heads_bwd(*[one] * 8, *dims, None) == 1
 
 
 def test_a_bias_that_broadcasts_stays_separate(monkeypatch):
