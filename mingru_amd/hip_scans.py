@@ -48,11 +48,17 @@ __all__ = [
     "block_step_impl",
     "workspace_errors",
     "LookbackError",
+    "KernelFailure",
 ]
 
 
 class ScanFallback(Exception):
     """The HIP path declines this call; the seam falls back to eager (or raises)."""
+
+
+class KernelFailure(ScanFallback):
+    """A call inside its envelope that failed all the same (a launch, an allocation): a
+    decline that is never passed over in silence."""
 
 
 # Block sizes the matrix kernels are compiled for (k x k transitions, k x v
@@ -316,13 +322,13 @@ def _same_device(*ts: torch.Tensor) -> None:
 
 
 def _funnel(what: str, fn, *args):
-    """Run ``fn`` and turn any launch-side failure into ``ScanFallback``."""
+    """Run ``fn`` and turn any launch-side failure into a ``ScanFallback`` (``KernelFailure``)."""
     try:
         return fn(*args)
     except (ScanFallback, LookbackError):
         raise
     except Exception as exc:  # noqa: BLE001 - every launch failure becomes a decline
-        raise ScanFallback(f"{what} HIP kernel failed: {exc}") from exc
+        raise KernelFailure(f"{what} HIP kernel failed: {exc}") from exc
 
 
 # ---------------------------------------------------------------------------
@@ -1807,6 +1813,10 @@ _BLOCK_STEP_MAX_B = 256
 _BLOCK_STEP_MAX_ELEMENTS = 64 * 768
 _BLOCK_STEP_GROUP = 16
 _BLOCK_STEP_MAX_LDS = 64 << 10
+# What the C entries take: elements of a row, rows of a projection, projections of a call.
+_BLOCK_STEP_MAX_ROW = 1 << 20
+_BLOCK_STEP_MAX_ROWS = 1 << 24
+_BLOCK_STEP_MAX_PROJECTIONS = 16
 
 
 def _step_project(x, ln, linears, rows, epi: int, res, out, dtype: int) -> None:
@@ -1874,6 +1884,10 @@ def block_step_impl(kind: str, x, ln1, proj, h_prev, gamma, delta, ln2, mlp):
         fits = fits and gamma.shape == (B, H if delta else d) and gamma.device == x.device
     if not fits or h_prev.shape != (B, width):
         raise ScanFallback(f"block step: shapes of the parts disagree at width {d}")
+    if (mlp and up[0] > _BLOCK_STEP_MAX_ROW) or (delta and (
+            inner > _BLOCK_STEP_MAX_ROW or H * dk > _BLOCK_STEP_MAX_ROWS
+            or len(rows) > _BLOCK_STEP_MAX_PROJECTIONS or max(dk, dv) > _DELTA_MAX_DIM)):
+        raise ScanFallback("block step: past the kernels' size limits")
     if not x.is_cuda or inner % 4 or (mlp and up[0] % 4):
         raise ScanFallback("block step: GPU tensors with rows of whole 4-element pieces")
     dev, dtype, index = x.device, x.dtype, x.get_device()

@@ -68,6 +68,7 @@ _warned_delta_decay_fallback = False
 _warned_gate_fallback = False
 _warned_mingru_gate_fallback = False
 _warned_step_fallback = False
+_warned_joined_failure = False
 
 # DeltaMinGRU ``auto`` region.  The HIP chunked-WY kernel beats the eager GPU
 # loop from a handful of chunks upward at every head size of its envelope, so
@@ -345,6 +346,13 @@ def _is_plain(m: nn.Module, cls: type) -> bool:
     )
 
 
+def _weight_bias(m: nn.Module):
+    """``(m.weight, m.bias)``, without the attribute look-ups of a module (half a microsecond
+    each, on every layer of every call) where they are registered as such."""
+    p = m._parameters
+    return p["weight"] if "weight" in p else m.weight, p["bias"] if "bias" in p else m.bias
+
+
 def _join_backend(x: torch.Tensor, linears, widths, impl: str):
     """The backend, if it has ``impl`` and one joined projection of ``x`` may stand in for
     ``linears`` of ``widths`` outputs; else ``None``.
@@ -370,7 +378,7 @@ def _join_backend(x: torch.Tensor, linears, widths, impl: str):
     for m, width in zip(linears, widths):
         if not _is_plain(m, nn.Linear):
             return None
-        w, b = m.weight, m.bias
+        w, b = _weight_bias(m)
         if w.shape != (width, columns) or (b is not None and b.shape != (width,)):
             return None
         this = (w.dtype, w.device, w.requires_grad,
@@ -389,8 +397,29 @@ def _join_backend(x: torch.Tensor, linears, widths, impl: str):
 
 def _join_linears(x: torch.Tensor, linears) -> torch.Tensor:
     """The outputs of ``linears`` on ``x`` side by side, from one product."""
-    bias = None if linears[0].bias is None else torch.cat([m.bias for m in linears])
-    return F.linear(x, torch.cat([m.weight for m in linears]), bias)
+    weights, biases = zip(*map(_weight_bias, linears))
+    return F.linear(x, torch.cat(weights), None if biases[0] is None else torch.cat(biases))
+
+
+def _try_joined(what: str, is_cuda: bool, backend, call):
+    """``call()`` of a joined form, or ``None`` for the separate projections: silently where
+    the kernels don't take the call.  A kernel that failed follows the mode's rules: the
+    forcing mode raises, ``auto`` warns once."""
+    try:
+        return call()
+    except backend.ScanFallback as exc:
+        if not isinstance(exc, getattr(backend, "KernelFailure", ())):
+            return None
+        mode = _resolve_scan_mode(is_cuda)
+        if mode != "auto":
+            raise RuntimeError(f"MINGRU_SCAN={mode} requested for {what}: {exc}") from exc
+        reason = str(exc)
+    global _warned_joined_failure
+    if not _warned_joined_failure:
+        warnings.warn(f"MINGRU_SCAN=auto ran the separate projections in place of {what}: {reason}",
+                      stacklevel=4)
+        _warned_joined_failure = True
+    return None
 
 
 def _dispatch_joined_gate_scan(kind: str, x, linears, width, h0, dt=None, lam=None,
@@ -398,7 +427,7 @@ def _dispatch_joined_gate_scan(kind: str, x, linears, width, h0, dt=None, lam=No
     """The fused gate scan from one joined projection of ``x`` (``width`` columns per layer),
     or ``None``.
 
-    ``None`` (silent in every mode) leads to the separate projections and
+    ``None`` (silent in every mode, ``_try_joined``) leads to the separate projections and
     ``_dispatch_signed_gate_scan`` / ``_dispatch_mingru_gate_scan``, which apply the
     mode's rules.  ``h0`` ``None`` starts every sequence at ``h0_const``.
     """
@@ -414,11 +443,9 @@ def _dispatch_joined_gate_scan(kind: str, x, linears, width, h0, dt=None, lam=No
     backend = _join_backend(x, linears, (width,) * len(linears), "gate_scan_packed_impl")
     if backend is None:
         return None
-    try:
-        return backend.gate_scan_packed_impl(kind, _join_linears(x, linears), h0, dt, lam,
-                                             h0_const=h0_const)
-    except backend.ScanFallback:
-        return None
+    return _try_joined("the joined gate scan", x.is_cuda, backend, lambda: (
+        backend.gate_scan_packed_impl(kind, _join_linears(x, linears), h0, dt, lam,
+                                      h0_const=h0_const)))
 
 
 def _dispatch_step(what: str, is_cuda: bool, call):
@@ -472,7 +499,7 @@ def _block_step_plan(block: nn.Module):
         out = mixer.out_proj
         if not _is_plain(out, nn.Linear):
             return None
-        delta = (mixer.n_heads, mixer.nh, mixer.d_k, mixer.d_v, (out.weight, out.bias))
+        delta = (mixer.n_heads, mixer.nh, mixer.d_k, mixer.d_v, _weight_bias(out))
     norms, mlp = [norm1], None
     if block.mlp is not None:
         seq = block.mlp
@@ -482,20 +509,25 @@ def _block_step_plan(block: nn.Module):
                 and _is_plain(seq[0], nn.Linear) and _is_plain(seq[3], nn.Linear)):
             return None
         norms.append(block.norm2)
-        mlp = ((seq[0].weight, seq[0].bias), (seq[3].weight, seq[3].bias))
+        mlp = (_weight_bias(seq[0]), _weight_bias(seq[3]))
+    ln = []
     for m in norms:
-        if not _is_plain(m, nn.LayerNorm) or m.weight is None or m.bias is None:
+        if not _is_plain(m, nn.LayerNorm):
             return None
+        w, b = _weight_bias(m)
+        if w is None or b is None:
+            return None
+        ln.append((w, b, m.eps))
     if not all(_is_plain(m, nn.Linear) for m in linears):
         return None
-    ln = [(m.weight, m.bias, m.eps) for m in norms]
-    return (kind, ln[0], [(m.weight, m.bias) for m in linears], delta,
+    return (kind, ln[0], [_weight_bias(m) for m in linears], delta,
             ln[1] if mlp else None, mlp)
 
 
 def _dispatch_block_step(block: nn.Module, x_t, h_prev, delta_t):
     """A whole residual block's decode step in a few launches, or ``None`` (silent in
-    every mode) for the layer-by-layer step, whose seams apply the mode's rules."""
+    every mode) for the layer-by-layer step, whose seams apply the mode's rules.  A launch
+    that fails raises, as it does in the layers' own step kernels."""
     if (_resolve_scan_mode(x_t.is_cuda) is None or x_t.dim() != 2
             or torch.is_autocast_enabled() or torch.nn.modules.module._has_any_global_hook()):
         return None
@@ -532,7 +564,7 @@ def _dispatch_block_step(block: nn.Module, x_t, h_prev, delta_t):
         return None
     try:
         return backend.block_step_impl(kind, x_t, ln1, proj, h_prev, gamma, delta, ln2, mlp)
-    except (backend.ScanFallback, RuntimeError):
+    except backend.ScanFallback:
         return None
 
 
@@ -1394,11 +1426,9 @@ class GivensMinGRU(DecayMixin, nn.Module):
             return None
         B, T, _ = x.shape
         gamma = self._decay_gamma(dt).expand(B, T, self.n_blocks) if dt is not None else None
-        try:
-            return backend.angle_joined_scan_impl(_join_linears(x, linears), gamma, h0_blocks,
-                                                  self.rounds)
-        except backend.ScanFallback:
-            return None
+        return _try_joined("the joined angle scan", x.is_cuda, backend, lambda: (
+            backend.angle_joined_scan_impl(_join_linears(x, linears), gamma, h0_blocks,
+                                           self.rounds)))
 
     def _angle_fused_forward(self, x, h0_blocks, dt):
         if not _angle_scan_should_try(x.is_cuda):
@@ -1613,16 +1643,18 @@ class DeltaMinGRU(DecayMixin, nn.Module):
                 tokens=x.shape[0] * x.shape[1], n_heads=self.n_heads, d_k=self.d_k,
                 d_v=self.d_v, nh=self.nh, chunk_size=self.chunk_size) is not None:
             return None
-        try:
+
+        def call():
             heads = backend.delta_heads_impl(_join_linears(x, linears), self.n_heads, self.nh,
                                              self.d_k, self.d_v)
             if log_gamma is None:
-                y, H_T = backend.delta_scan_impl(*heads, H, chunk_size=self.chunk_size)
-            else:
-                y, H_T = backend.delta_gated_scan_impl(*heads, log_gamma, H,
-                                                       chunk_size=self.chunk_size)
-        except backend.ScanFallback:
+                return backend.delta_scan_impl(*heads, H, chunk_size=self.chunk_size)
+            return backend.delta_gated_scan_impl(*heads, log_gamma, H, chunk_size=self.chunk_size)
+
+        scanned = _try_joined("the joined DeltaMinGRU path", x.is_cuda, backend, call)
+        if scanned is None:
             return None
+        y, H_T = scanned
         return y.permute(0, 2, 1, 3), H_T
 
     def _delta_gated_fused_forward(self, x, H, dt):
