@@ -19,11 +19,13 @@ __device__ __forceinline__ float mg_sigmoid(float x) {
 }
 __device__ __forceinline__ float mg_tanh(float x) { return fmaf(2.f, mg_sigmoid(2.f * x), -1.f); }
 // sigmoid(x) and sigmoid(-x) from one exponential: with e = e^-|x| in (0, 1],
-// sigmoid(|x|) = 1 / (1 + e) and sigmoid(-|x|) = e / (1 + e), so neither overflows and
-// both keep the relative error of mg_sigmoid (an exp2 and a reciprocal, one rounding more).
+// sigmoid(|x|) = 1 / (1 + e) and sigmoid(-|x|) = e / (1 + e), so neither overflows.  The
+// second is the quotient corrected by its remainder: as the plain product of e and the
+// reciprocal it carried both their roundings and its own.
 __device__ __forceinline__ void mg_sigmoid_pair(float x, float& pos, float& neg) {
   const float e = __builtin_amdgcn_exp2f(-1.44269504088896341f * fabsf(x));
-  const float big = __builtin_amdgcn_rcpf(1.f + e), small = e * big;
+  const float d = 1.f + e, big = __builtin_amdgcn_rcpf(d), q = e * big;
+  const float small = fmaf(big, fmaf(-d, q, e), q);
   pos = x >= 0.f ? big : small;
   neg = x >= 0.f ? small : big;
 }

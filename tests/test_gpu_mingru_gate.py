@@ -197,3 +197,22 @@ def test_small_problem_two_launch_form(cuda, case, monkeypatch):
     shapes run as one launch whose workgroups fold their predecessors' aggregates."""
     monkeypatch.setenv("MINGRU_HIP_EW_FORM", "two")
     test_mingru_gate_scan_matches_fp64(cuda, case)
+
+
+def test_gate_pair_keeps_the_error_of_one_sigmoid(cuda):
+    """Both gates come from one exponential.  Over |k| < 1 the smaller of the two is no
+    further from float64 (root mean square, 10% for the chance part of a million points)
+    than the larger, which is a plain reciprocal: as the product of the exponential and that
+    reciprocal it was 21% further off.  Written gate by gate: h = z with g = 1 and h0 = 0,
+    h = a with g = 0 and h0 = 1."""
+    print("[gpu] MinGRU gate pair against float64", flush=True)
+    k = torch.linspace(-1, 1, 1_000_001, device=cuda)[None, None]
+    low = torch.full_like(k, -200.0)  # g(low) = e^low = 0
+    z = hip_scans.mingru_gate_scan_impl(k, torch.full_like(k, 0.5), low)
+    a = hip_scans.mingru_gate_scan_impl(k, low, torch.zeros_like(k))
+    for got, x in ((z, k), (a, -k)):
+        ref = torch.sigmoid(x.double())
+        off = ((got.double() - ref) / ref) ** 2
+        small, large = (off[m].mean().sqrt().item() for m in (x < 0, x > 0))
+        assert large <= 6e-8  # one ulp of the reciprocal
+        assert small <= 1.1 * large, f"{small:.2e} against {large:.2e}"
