@@ -27,6 +27,7 @@ other three scans (reference ``:755-807, 1454-1655``).
 
 from __future__ import annotations
 
+import functools
 import math
 import os
 import warnings
@@ -35,6 +36,7 @@ from typing import Literal
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd.function import once_differentiable
 
 __all__ = [
     "MinGRU",
@@ -357,8 +359,8 @@ def _join_backend(x: torch.Tensor, linears, widths, impl: str):
     """The backend, if it has ``impl`` and one joined projection of ``x`` may stand in for
     ``linears`` of ``widths`` outputs; else ``None``.
 
-    Joined, the projections are one matrix product each way instead of one per layer, and
-    the input's gradient needs no sum (fwd+bwd of three 1024-wide bf16 projections of 16384
+    Joined, the projections are one matrix product each way instead of one per layer (fp32:
+    forward, and ``_JoinedLinear`` back), and the input's gradient needs no sum (fwd+bwd of three 1024-wide bf16 projections of 16384
     rows: 614 -> 360 us).  Only for what calling each layer would compute anyway: plain
     ``nn.Linear`` modules without hooks, of the widths that the joined rows are split at,
     alike in dtype, device, bias and whether they are trained.
@@ -395,10 +397,84 @@ def _join_backend(x: torch.Tensor, linears, widths, impl: str):
     return backend
 
 
+# Outputs of a layer below which its weight's gradient is a product of its own in fp32: the
+# library splits such a product over the rows, so its sums are shorter (DeltaMinGRU's beta
+# layers, 4 to 16 outputs: error against float64 1.4 to 1.6 times larger side by side).
+_JOIN_NARROW = 64
+
+
+@functools.lru_cache(maxsize=256)
+def _join_spans(widths: tuple):
+    """How the backward of layers of ``widths`` side by side splits their columns: for the
+    input's gradient into wide layers with the narrow ones after each, for the weights'
+    gradients into runs of wide layers and single narrow ones (the layers of each span)."""
+    inputs, weights, wide = [], [], False
+    for n in widths:
+        narrow = n < _JOIN_NARROW
+        if inputs and narrow:
+            inputs[-1] += n
+        else:
+            inputs.append(n)
+        if wide and not narrow:
+            weights[-1].append(n)
+        else:
+            weights.append([n])
+        wide = not narrow
+    return inputs, [sum(span) for span in weights], weights
+
+
+class _JoinedLinear(torch.autograd.Function):
+    """fp32 layers side by side: one product forward, and a backward whose sums are no longer
+    than the separate layers'.
+
+    As one product, the input's gradient sums over every layer's outputs at once; its error
+    against float64 was 1.05 to 1.19 times the separate layers' (two to three layers of 64
+    to 1024 outputs).  bf16 layers stay one product each way: there the separate gradients'
+    roundings outweigh it (0.73 to 0.82 times the error joined).
+    """
+
+    @staticmethod
+    def forward(ctx, x, widths, *params):
+        n = len(widths)
+        W = torch.cat(params[:n])
+        ctx.save_for_backward(x, W)
+        ctx.widths = widths
+        return F.linear(x, W, torch.cat(params[n:]) if len(params) > n else None)
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dP):
+        x, W = ctx.saved_tensors
+        need, widths = ctx.needs_input_grad, ctx.widths
+        n = len(widths)
+        rows = dP.reshape(-1, W.shape[0])
+        inputs, spans, layers = _join_spans(widths)
+        dx, dws, dbs = None, [None] * n, [None] * (len(need) - 2 - n)
+        if need[0]:
+            for part, w in zip(rows.split(inputs, 1), W.split(inputs)):
+                dx = part @ w if dx is None else dx.addmm_(part, w)
+            dx = dx.view(x.shape)
+        if need[2]:
+            cols, dws = x.reshape(-1, W.shape[1]), []
+            for part, span in zip(rows.t().split(spans), layers):
+                dw = part @ cols
+                dws += dw.split(span) if len(span) > 1 else (dw,)
+        if dbs and need[2 + n]:
+            dbs = rows.sum(0).split(widths)
+        return dx, None, *dws, *dbs
+
+
 def _join_linears(x: torch.Tensor, linears) -> torch.Tensor:
     """The outputs of ``linears`` on ``x`` side by side, from one product."""
     weights, biases = zip(*map(_weight_bias, linears))
-    return F.linear(x, torch.cat(weights), None if biases[0] is None else torch.cat(biases))
+    biases = () if biases[0] is None else biases
+    if (weights[0].dtype == torch.float32 and torch.is_grad_enabled()
+            and not torch.is_autocast_enabled()):
+        try:
+            return _JoinedLinear.apply(x, tuple(w.shape[0] for w in weights), *weights, *biases)
+        except RuntimeError:
+            pass  # a transform that takes no Python function (forward mode, vmap)
+    return F.linear(x, torch.cat(weights), torch.cat(biases) if biases else None)
 
 
 def _try_joined(what: str, is_cuda: bool, backend, call):

@@ -351,3 +351,81 @@ def test_joined_equals_separate_under_autocast(cuda, case, monkeypatch):
                 f"output {i}: joined {_off(a, r):.2e}, separate {_off(b, r):.2e} off float64")
         else:
             assert torch.equal(a, b), f"output {i}"
+
+
+# fp32 layers whose joined backward could sum in another order than the separate one:
+# inputs of one long product against several short ones, weights of a few columns.
+PRECISION = [
+    (lambda: DeltaMinGRU(256, 256, n_heads=4), 8, 1000),
+    (lambda: DeltaMinGRU(256, 256, n_heads=4, nh=2), 4, 1500),
+    (lambda: SignedMinGRU(320, 320), 8, 500),
+    (lambda: MinGRU(256, 512), 4, 700),
+    (lambda: GivensMinGRU(256, 512), 4, 500),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", range(len(PRECISION)))
+def test_joined_gradients_lose_no_precision(cuda, case, monkeypatch):
+    """No fp32 gradient is further from float64 joined than separate.  3% is the chance part:
+    the smallest outputs compared have some thousand entries.  (The biases, a handful of
+    entries in places, are held by the comparison above.)"""
+    build, B, T = PRECISION[case]
+    print(f"[gpu] joined precision case={case}", flush=True)
+    torch.manual_seed(7 + case)
+    joined, separate = _pair(cuda, build(), torch.float32)
+    x = torch.randn(B, T, joined.input_size, device=cuda)
+    gy = None
+    res = []
+    for m, mode in ((joined, "hip"), (separate, "hip"), (copy.deepcopy(separate).double(), "eager")):
+        monkeypatch.setenv("MINGRU_SCAN", mode)
+        xi = x.to(next(m.parameters()).dtype).requires_grad_()
+        y = m(xi)
+        gy = torch.randn(y.shape, generator=torch.Generator().manual_seed(9)).to(cuda) \
+            if gy is None else gy
+        names = [n for n, _ in m.named_parameters() if n.endswith("weight")]
+        grads = torch.autograd.grad(y, [xi, *(m.get_parameter(n) for n in names)], gy.to(y.dtype))
+        res.append(grads)
+    for n, a, b, r in zip(["x", *names], *res):
+        assert _off(a, r) <= 1.03 * _off(b, r), (
+            f"{n}: joined {_off(a, r):.3e}, separate {_off(b, r):.3e} off float64")
+
+
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("x_grad,w_grad,b_grad", [(True, True, True), (False, True, False),
+                                                  (True, False, False), (False, False, True)])
+def test_joined_linears_differentiate(bias, x_grad, w_grad, b_grad):
+    """The joined projection's own backward: every layer's gradients, layers of a few
+    columns and wide ones in any order, each only where it is asked for."""
+    torch.manual_seed(2)
+    linears = [nn.Linear(12, n, bias=bias) for n in (70, 64, 3, 80, 1)]
+    for m in linears:
+        m.weight.requires_grad_(w_grad)
+        if bias:
+            m.bias.requires_grad_(b_grad)
+    x = torch.randn(2, 9, 12, requires_grad=x_grad)
+    leaves = [t for t in (x, *(p for m in linears for p in m.parameters())) if t.requires_grad]
+    if not leaves:
+        return
+    P, want = mg._join_linears(x, linears), torch.cat([m(x) for m in linears], -1)
+    torch.testing.assert_close(P, want)
+    g = torch.randn_like(P)
+    for a, b in zip(torch.autograd.grad(P, leaves, g), torch.autograd.grad(want, leaves, g)):
+        assert a.shape == b.shape and a.dtype == b.dtype
+        torch.testing.assert_close(a, b)
+
+
+def test_joined_linears_under_transforms():
+    """Forward mode and vmap, which take no Python function, take the plain product."""
+    torch.manual_seed(3)
+    linears = [nn.Linear(6, n) for n in (66, 2)]
+    x, t = torch.randn(2, 4, 6), torch.randn(2, 4, 6)
+
+    def separate(x):
+        return torch.cat([m(x) for m in linears], -1)
+
+    got = torch.func.jvp(lambda x: mg._join_linears(x, linears), (x,), (t,))
+    torch.testing.assert_close(got, torch.func.jvp(separate, (x,), (t,)))
+    torch.testing.assert_close(torch.func.vmap(lambda x: mg._join_linears(x, linears))(x), separate(x))
+    torch.testing.assert_close(torch.func.grad(lambda x: mg._join_linears(x, linears).sum())(x),
+                               torch.func.grad(lambda x: separate(x).sum())(x))
