@@ -18,6 +18,7 @@ import types
 import pytest
 import torch
 from torch import nn
+from torch.utils._python_dispatch import TorchDispatchMode
 
 import mingru_amd
 from mingru_amd import DeltaMinGRU, GivensMinGRU, MinGRU, SignedMinGRU
@@ -413,6 +414,52 @@ def test_joined_linears_differentiate(bias, x_grad, w_grad, b_grad):
     for a, b in zip(torch.autograd.grad(P, leaves, g), torch.autograd.grad(want, leaves, g)):
         assert a.shape == b.shape and a.dtype == b.dtype
         torch.testing.assert_close(a, b)
+
+
+class _Products(TorchDispatchMode):
+    """Counts the multiply-adds of matrix products and the reductions run inside."""
+
+    def __init__(self):
+        super().__init__()
+        self.work = self.sums = 0
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        if func.overloadpacket in (torch.ops.aten.mm, torch.ops.aten.addmm_):
+            a, b = args[-2:]
+            self.work += a.shape[0] * a.shape[1] * b.shape[1]
+        self.sums += func is torch.ops.aten.sum.dim_IntList
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("leaf", [True, False])
+@pytest.mark.parametrize("how", ["grad", "backward"])
+def test_joined_linears_form_what_is_asked_for(how, leaf):
+    """The input's gradient, the weights' and the biases' are each formed only if any of
+    them is asked for."""
+    torch.manual_seed(4)
+    linears = [nn.Linear(12, n) for n in (70, 64, 3, 80)]
+    x = torch.randn(18, 12, requires_grad=True)
+    if not leaf:
+        x = 2 * x
+        x.retain_grad()
+    one = 18 * 12 * (70 + 64 + 3 + 80)
+    asked = [((linears[1].weight,), one, 0), ((x,), one, 0), ((linears[2].bias,), 0, 1),
+             ((x, *(m.weight for m in linears)), 2 * one, 0),
+             ((x, linears[0].bias, linears[3].weight), 2 * one, 1)]
+    for leaves, work, sums in asked:
+        P, want = mg._join_linears(x, linears), torch.cat([m(x) for m in linears], -1)
+        g = torch.randn_like(P)
+        with _Products() as count:
+            if how == "grad":
+                got = torch.autograd.grad(P, leaves, g, retain_graph=True)
+            else:
+                for t in leaves:
+                    t.grad = None
+                P.backward(g, inputs=list(leaves), retain_graph=True)
+                got = [t.grad for t in leaves]
+        assert (count.work, count.sums) == (work, sums)
+        for a, b in zip(got, torch.autograd.grad(want, leaves, g, retain_graph=True)):
+            torch.testing.assert_close(a, b)
 
 
 def test_joined_linears_under_transforms():
