@@ -2,7 +2,7 @@
 
 Reference: the recurrence in float64 on the bf16 inputs, differentiated by torch
 autograd.  The kernels compute in fp32 and round each output once, so an output x may
-be off by bf16's unit roundoff 2^-9 |x| plus the fp32 kernels' own bars (1e-4 forward,
+be off by bf16's unit roundoff 2^-8 |x| plus the fp32 kernels' own bars (1e-4 forward,
 1e-3 gradients); a recorded fp32 state that had been rounded to bf16 would exceed it.
 """
 

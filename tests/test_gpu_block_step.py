@@ -57,12 +57,17 @@ def test_block_step(cuda, case, given_state, dtype, monkeypatch):
     h = _state(case, cuda, dtype, g) if given_state else None
     dt = torch.rand(B, generator=g).to(cuda, dtype) if kw.get("decay") else None
     calls = []
-    real = hip_scans.block_step_impl
-    monkeypatch.setattr(hip_scans, "block_step_impl", lambda *a: calls.append(1) or real(*a))
+    real = hip_scans._call
+    monkeypatch.setattr(hip_scans, "_call",
+                        lambda name, *a: (real(name, *a), calls.append(name)))
     y, s = fused.step(x, h, dt)
-    assert calls == [1], "the fused step did not run"
+    launches = ["mg_step_gate"] if mixer != "delta" else [
+        "mg_step_project", "mg_delta_step_heads", "mg_step_project"]
+    launches += ["mg_step_project"] * (2 if exp else 0)
+    assert calls == launches, "the fused step did not run"
+    calls.clear()
     yl, sl = layers.step(x, h, dt)
-    assert calls == [1]
+    assert calls == ["mg_delta_step" if mixer == "delta" else "mg_gate_step"]
     monkeypatch.setenv("MINGRU_SCAN", "eager")
     ref = copy.deepcopy(fused).double()
     yr, sr = ref.step(x.double(), None if h is None else h.double(),
