@@ -360,10 +360,11 @@ def _join_backend(x: torch.Tensor, linears, widths, impl: str):
     ``linears`` of ``widths`` outputs; else ``None``.
 
     Joined, the projections are one matrix product each way instead of one per layer (fp32:
-    forward, and ``_JoinedLinear`` back), and the input's gradient needs no sum (fwd+bwd of three 1024-wide bf16 projections of 16384
-    rows: 614 -> 360 us).  Only for what calling each layer would compute anyway: plain
-    ``nn.Linear`` modules without hooks, of the widths that the joined rows are split at,
-    alike in dtype, device, bias and whether they are trained.
+    forward, and ``_JoinedLinear`` back), and the input's gradient needs no sum (fwd+bwd of
+    three 1024-wide bf16 projections of 16384 rows: 614 -> 360 us).  Only for what calling
+    each layer would compute anyway: plain ``nn.Linear`` modules without hooks, of the widths
+    that the joined rows are split at, alike in dtype, device, bias and whether they are
+    trained.
     """
     rows = x.numel() // max(1, x.shape[-1])
     if not torch.is_grad_enabled() and rows < _JOIN_MIN_ROWS:
@@ -402,45 +403,63 @@ def _join_backend(x: torch.Tensor, linears, widths, impl: str):
 # layers, 4 to 16 outputs: error against float64 1.4 to 1.6 times larger side by side).
 _JOIN_NARROW = 64
 
+# Multiply-adds of a joined bf16 product from which its backward asks which weights'
+# gradients are wanted.  Forward and one weight's gradient of SignedMinGRU: 374 -> 324 us at
+# 16384 rows of 3 x 1024 outputs (48 Gi; separate layers 339); with half the rows the Python
+# function's host time outweighs the products saved (267 -> 308, separate layers 331).
+_JOIN_ASK_WORK = 1 << 35
 
 @functools.lru_cache(maxsize=256)
-def _join_spans(widths: tuple):
-    """How the backward of layers of ``widths`` side by side splits their columns: for the
-    input's gradient into wide layers with the narrow ones after each, for the weights'
-    gradients into runs of wide layers and single narrow ones."""
-    inputs, weights, wide = [], [], False
+def _join_spans(widths: tuple, narrow: int):
+    """How the input's gradient splits the columns of layers of ``widths`` side by side: wide
+    layers with the ones below ``narrow`` columns after each."""
+    spans = []
     for n in widths:
-        narrow = n < _JOIN_NARROW
-        if inputs and narrow:
-            inputs[-1] += n
+        if spans and n < narrow:
+            spans[-1] += n
         else:
-            inputs.append(n)
-        if wide and not narrow:
-            weights[-1] += n
+            spans.append(n)
+    return spans
+
+
+@functools.lru_cache(maxsize=256)
+def _join_weight_spans(widths: tuple, asked: tuple, narrow: int):
+    """The same for the weights' gradients, and which are asked for: runs of wide layers
+    alike in that, and single narrow ones."""
+    spans, wanted, last = [], [], None
+    for n, a in zip(widths, asked):
+        kind = None if a and n < narrow else a
+        if spans and kind is not None and kind == last:
+            spans[-1] += n
         else:
-            weights.append(n)
-        wide = not narrow
-    return inputs, weights
+            spans.append(n)
+            wanted.append(a)
+        last = kind
+    return spans, wanted
 
 
 _will_execute = getattr(torch._C, "_will_engine_execute_node", None)
 
 
-def _asked_for(ctx) -> list:
-    """Which tensor inputs of a Python function the running backward needs a gradient for
-    (``needs_input_grad`` only says which are trained at all).  None of them may be a leaf:
-    for a leaf that ``torch.autograd.grad`` was given the engine raises instead."""
-    return [node is not None and (_will_execute is None or _will_execute(node))
-            for node, _ in ctx.next_functions]
+def _asked(node) -> bool:
+    """Whether the running backward needs a gradient that goes to ``node``
+    (``needs_input_grad`` of a Python function only says which inputs are trained at all)."""
+    if node is None or _will_execute is None:
+        return node is not None
+    try:
+        return _will_execute(node)
+    except RuntimeError:  # how the engine answers for a leaf that torch.autograd.grad was given
+        return True
 
 
 class _JoinedLinear(torch.autograd.Function):
-    """fp32 layers of ``widths`` outputs side by side, ``x W^T + bias``: one product forward,
-    and a backward whose sums are no longer than the separate layers'.
+    """Layers of ``widths`` outputs side by side, ``x W^T + bias``: one product forward, and a
+    backward that forms only the gradients that are asked for, in fp32 in sums no longer than
+    the separate layers'.
 
     As one product, the input's gradient sums over every layer's outputs at once; its error
-    against float64 was 1.05 to 1.19 times the separate layers' (two to three layers of 64
-    to 1024 outputs).  bf16 layers stay one product each way: there the separate gradients'
+    against float64 was 1.05 to 1.19 times the separate layers' (fp32, two to three layers of
+    64 to 1024 outputs).  bf16 layers stay one product each way: there the separate gradients'
     roundings outweigh it (0.73 to 0.82 times the error joined).
     """
 
@@ -454,29 +473,39 @@ class _JoinedLinear(torch.autograd.Function):
     @once_differentiable
     def backward(ctx, dP):
         x, W = ctx.saved_tensors
-        need_x, need_w, *need_b = _asked_for(ctx)
-        inputs, spans = _join_spans(ctx.widths)
+        x_node, cat, *biases = (node for node, _ in ctx.next_functions)
         rows = dP.reshape(-1, W.shape[0])
         dx = dW = None
-        if need_x:
+        exact = W.dtype == torch.float32
+        narrow = _JOIN_NARROW if exact else 0
+        if _asked(x_node):
+            inputs = _join_spans(ctx.widths, narrow) if exact else [W.shape[0]]
             for part, w in zip(rows.split(inputs, 1), W.split(inputs)):
                 dx = part @ w if dx is None else dx.addmm_(part, w)
             dx = dx.view(x.shape)
-        if need_w:
+        if _asked(cat):
+            layers = tuple(_asked(node) for node, _ in cat.next_functions)
+            spans, asked = _join_weight_spans(ctx.widths, layers, narrow)
             cols, dW = x.reshape(-1, W.shape[1]), torch.empty_like(W)
-            for part, dw in zip(rows.t().split(spans), dW.split(spans)):
-                torch.mm(part, cols, out=dw)
-        return dx, dW, rows.sum(0) if any(need_b) else None, None
+            for part, dw, wanted in zip(rows.t().split(spans), dW.split(spans), asked):
+                if wanted:
+                    torch.mm(part, cols, out=dw)
+                else:
+                    dw.zero_()
+        return dx, dW, rows.sum(0) if any(map(_asked, biases)) else None, None
 
 
 def _join_linears(x: torch.Tensor, linears) -> torch.Tensor:
     """The outputs of ``linears`` on ``x`` side by side, from one product."""
     weights, biases = zip(*map(_weight_bias, linears))
+    widths = tuple(w.shape[0] for w in weights)
+    exact = weights[0].dtype == torch.float32
+    ask = torch.is_grad_enabled() and not torch.is_autocast_enabled() and (
+        exact or x.numel() * sum(widths) >= _JOIN_ASK_WORK)
     W, bias = torch.cat(weights), None if biases[0] is None else torch.cat(biases)
-    if W.dtype == torch.float32 and torch.is_grad_enabled() and not torch.is_autocast_enabled():
+    if ask:
         try:
-            return _JoinedLinear.apply(x.view_as(x) if x.is_leaf else x, W, bias,
-                                       tuple(w.shape[0] for w in weights))
+            return _JoinedLinear.apply(x, W, bias, widths)
         except RuntimeError:
             pass  # a transform that takes no Python function (forward mode, vmap)
     return F.linear(x, W, bias)

@@ -471,19 +471,22 @@ class _Products(TorchDispatchMode):
 
 @pytest.mark.parametrize("leaf", [True, False])
 @pytest.mark.parametrize("how", ["grad", "backward"])
-def test_joined_linears_form_what_is_asked_for(how, leaf):
-    """The input's gradient, the weights' and the biases' are each formed only if any of
-    them is asked for."""
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_joined_linears_form_what_is_asked_for(how, leaf, dtype, monkeypatch):
+    """The input's gradient and each weight's are formed only if they are asked for, the
+    biases' if any of them is: always in fp32, in bf16 past a size (here: any)."""
+    monkeypatch.setattr(mg, "_JOIN_ASK_WORK", 0)
     torch.manual_seed(4)
-    linears = [nn.Linear(12, n) for n in (70, 64, 3, 80)]
-    x = torch.randn(18, 12, requires_grad=True)
+    linears = [nn.Linear(12, n, dtype=dtype) for n in (70, 64, 3, 80)]
+    x = torch.randn(18, 12, dtype=dtype, requires_grad=True)
     if not leaf:
         x = 2 * x
         x.retain_grad()
     one = 18 * 12 * (70 + 64 + 3 + 80)
-    asked = [((linears[1].weight,), one, 0), ((x,), one, 0), ((linears[2].bias,), 0, 1),
+    asked = [((linears[1].weight,), 18 * 12 * 64, 0), ((x,), one, 0), ((linears[2].bias,), 0, 1),
+             ((linears[0].weight, linears[2].weight), 18 * 12 * (70 + 3), 0),
              ((x, *(m.weight for m in linears)), 2 * one, 0),
-             ((x, linears[0].bias, linears[3].weight), 2 * one, 1)]
+             ((x, linears[0].bias, linears[3].weight), one + 18 * 12 * 80, 1)]
     for leaves, work, sums in asked:
         P, want = mg._join_linears(x, linears), torch.cat([m(x) for m in linears], -1)
         g = torch.randn_like(P)
@@ -497,7 +500,10 @@ def test_joined_linears_form_what_is_asked_for(how, leaf):
                 got = [t.grad for t in leaves]
         assert (count.work, count.sums) == (work, sums)
         for a, b in zip(got, torch.autograd.grad(want, leaves, g, retain_graph=True)):
-            torch.testing.assert_close(a, b)
+            # bf16: half a unit (2^-9) for each of the separate input gradient's four parts, of
+            # magnitude 2, and of their sums.
+            torch.testing.assert_close(a, b, **({} if dtype == torch.float32 else
+                                                dict(rtol=2.0**-6, atol=2.0**-6)))
 
 
 def test_joined_linears_under_transforms():
