@@ -1803,16 +1803,21 @@ def delta_step_impl(H, q, K, V, beta, log_gamma):
     return y.to(q.dtype), Hn.to(H.dtype)
 
 
-# Whole-block decode (csrc/decode_block.hip): sequences per call, sequences a workgroup
-# takes, and the bytes of their normalised inputs it holds.  Each group of 16 sequences
-# reads the weights again and the products run on the vector units, so past a batch times
-# width the library's matrix products are the better ones: three blocks of width 768 take
-# 211 us a token up to 32 sequences (host-bound), 279 at 64 and 507 at 128, layer by layer
-# 760 us of which about 300 are kernels.
+# Whole-block decode (csrc/decode_block.hip): sequences per call, elements of their inputs,
+# sequences a workgroup takes, the bytes of their normalised inputs it holds, and padded
+# sequences times the square of the width.  The products run on the vector units for a batch
+# padded to its tile, and each group of 16 sequences reads the weights again, so past that
+# product the library's matrix products are the better ones.  One SignedMinGRU block, fp32, us
+# a token eager (host-bound until the kernels pass about 150), fused / layer by layer:
+# 25 M: 512 wide, 96 sequences 61 / 155; 38 M: 768 x 64 85 / 157, 3072 x 4 145 / 158; 50 M:
+# 1024 x 48 128 / 155; 67 M: 4096 x 2 215 / 170, 8192 x 1 685 / 562; 75 M: 3072 x 5 232 / 157.
+# In kernels alone the layers are ahead from about 25 M on (60 / 60, 82 / 61, 143 / 125,
+# 123 / 67); below it 1024 x 16 62 / 64, 256 x 192 42 / 186.
 _BLOCK_STEP_MAX_B = 256
 _BLOCK_STEP_MAX_ELEMENTS = 64 * 768
 _BLOCK_STEP_GROUP = 16
 _BLOCK_STEP_MAX_LDS = 64 << 10
+_BLOCK_STEP_MAX_WORK = 48 << 20
 # What the C entries take: elements of a row, rows of a projection, projections of a call.
 _BLOCK_STEP_MAX_ROW = 1 << 20
 _BLOCK_STEP_MAX_ROWS = 1 << 24
@@ -1844,6 +1849,11 @@ def _projection_rows(pairs, K: int) -> list:
     return rows
 
 
+def _block_step_tiles(B: int) -> int:
+    """``B`` sequences padded to the kernels' tiles: 1, 4 or 8, or groups of 16."""
+    return next((n for n in (1, 4, 8) if B <= n), -(-B // _BLOCK_STEP_GROUP) * _BLOCK_STEP_GROUP)
+
+
 def block_step_impl(kind: str, x, ln1, proj, h_prev, gamma, delta, ln2, mlp):
     """One decode step of a residual block; returns ``(x_out, state)``.
 
@@ -1858,7 +1868,9 @@ def block_step_impl(kind: str, x, ln1, proj, h_prev, gamma, delta, ln2, mlp):
     B, d = x.shape
     if x.dtype not in (torch.float32, torch.bfloat16) or not 1 <= B <= _BLOCK_STEP_MAX_B:
         raise ScanFallback(f"block step: {x.dtype} x {tuple(x.shape)}")
-    if d % 4 or B * d > _BLOCK_STEP_MAX_ELEMENTS or 4 * min(B, _BLOCK_STEP_GROUP) * d > _BLOCK_STEP_MAX_LDS:
+    if (d % 4 or B * d > _BLOCK_STEP_MAX_ELEMENTS
+            or 4 * min(B, _BLOCK_STEP_GROUP) * d > _BLOCK_STEP_MAX_LDS
+            or _block_step_tiles(B) * d * d > _BLOCK_STEP_MAX_WORK):
         raise ScanFallback(f"block step: width {d} at {B} sequences")
     # Every shape the kernels take for granted: they read K elements of each row, and the
     # layers of an edited block may not fit together.

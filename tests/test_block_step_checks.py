@@ -61,3 +61,17 @@ def test_state_and_decay_of_another_shape_are_refused(mixer):
                      (torch.zeros(B, width), torch.zeros(B, 1))):
         with pytest.raises(hip_scans.ScanFallback, match="shape"):
             hip_scans.block_step_impl(kind, x, ln1, proj, h, gamma, delta, ln2, mlp)
+
+
+@pytest.mark.parametrize("d,b,taken", [
+    (4096, 1, True), (4096, 2, False), (8192, 1, False), (3072, 4, True), (3072, 5, False),
+    (2048, 8, True), (2048, 9, False), (1024, 48, True), (1024, 49, False), (256, 192, True),
+    (256, 193, False), (18, 2, False)])
+def test_sizes_that_the_layers_run_faster_are_declined(d, b, taken):
+    """Padded sequences times the square of the width bound the kernels' work, beside the
+    bounds on the input; the message tells the size's refusal from the CPU tensors'."""
+    meta = lambda *s: torch.empty(*s, device="meta")  # noqa: E731
+    ln, pair = (meta(d), meta(d), 1e-5), (meta(d, d), meta(d))
+    with pytest.raises(hip_scans.ScanFallback, match="GPU tensors" if taken else "width"):
+        hip_scans.block_step_impl("mingru", meta(b, d), ln, [pair] * 2, meta(b, d), None, None, None,
+                                  None)
