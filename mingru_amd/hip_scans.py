@@ -46,6 +46,7 @@ __all__ = [
     "delta_heads_impl",
     "delta_joined_reason",
     "block_step_impl",
+    "block_step_reason",
     "workspace_errors",
     "LookbackError",
     "KernelFailure",
@@ -1854,6 +1855,18 @@ def _block_step_tiles(B: int) -> int:
     return next((n for n in (1, 4, 8) if B <= n), -(-B // _BLOCK_STEP_GROUP) * _BLOCK_STEP_GROUP)
 
 
+def block_step_reason(B: int, d: int, dtype) -> str | None:
+    """Why ``block_step_impl`` would decline ``B`` sequences of width ``d``, asked before its
+    arguments are put together; ``None`` where it would not for their size and type."""
+    if dtype not in (torch.float32, torch.bfloat16) or not 1 <= B <= _BLOCK_STEP_MAX_B:
+        return f"block step: {B} sequences of {dtype}"
+    if (d % 4 or B * d > _BLOCK_STEP_MAX_ELEMENTS
+            or 4 * min(B, _BLOCK_STEP_GROUP) * d > _BLOCK_STEP_MAX_LDS
+            or _block_step_tiles(B) * d * d > _BLOCK_STEP_MAX_WORK):
+        return f"block step: width {d} at {B} sequences"
+    return None
+
+
 def block_step_impl(kind: str, x, ln1, proj, h_prev, gamma, delta, ln2, mlp):
     """One decode step of a residual block; returns ``(x_out, state)``.
 
@@ -1866,12 +1879,9 @@ def block_step_impl(kind: str, x, ln1, proj, h_prev, gamma, delta, ln2, mlp):
     (weight, bias) pairs.  All tensors share ``x``'s dtype, fp32 or bf16, and are dense.
     """
     B, d = x.shape
-    if x.dtype not in (torch.float32, torch.bfloat16) or not 1 <= B <= _BLOCK_STEP_MAX_B:
-        raise ScanFallback(f"block step: {x.dtype} x {tuple(x.shape)}")
-    if (d % 4 or B * d > _BLOCK_STEP_MAX_ELEMENTS
-            or 4 * min(B, _BLOCK_STEP_GROUP) * d > _BLOCK_STEP_MAX_LDS
-            or _block_step_tiles(B) * d * d > _BLOCK_STEP_MAX_WORK):
-        raise ScanFallback(f"block step: width {d} at {B} sequences")
+    reason = block_step_reason(B, d, x.dtype)
+    if reason is not None:
+        raise ScanFallback(reason)
     # Every shape the kernels take for granted: they read K elements of each row, and the
     # layers of an edited block may not fit together.
     rows, pairs, row, lns = _projection_rows(proj, d), [*proj], (d,), [*ln1[:2]]

@@ -647,6 +647,9 @@ def _dispatch_block_step(block: nn.Module, x_t, h_prev, delta_t):
         return None
     if not hasattr(backend, "block_step_impl") or backend.available() is not True:
         return None
+    if (not x_t.is_contiguous()
+            or backend.block_step_reason(x_t.size(0), x_t.size(1), x_t.dtype) is not None):
+        return None
     plan = _block_step_plan(block)
     if plan is None:
         return None

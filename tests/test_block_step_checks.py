@@ -75,3 +75,20 @@ def test_sizes_that_the_layers_run_faster_are_declined(d, b, taken):
     with pytest.raises(hip_scans.ScanFallback, match="GPU tensors" if taken else "width"):
         hip_scans.block_step_impl("mingru", meta(b, d), ln, [pair] * 2, meta(b, d), None, None, None,
                                   None)
+
+
+def test_a_size_that_is_declined_plans_nothing(monkeypatch):
+    """The dispatch looks at the input's size, type and layout before it walks the block's
+    modules, and takes the layers; for another input it goes on to the plan."""
+    plans = []
+    real = mg._block_step_plan
+    monkeypatch.setenv("MINGRU_SCAN", "hip")
+    monkeypatch.setattr(hip_scans, "available", lambda: True)
+    monkeypatch.setattr(mg, "_block_step_plan", lambda b: plans.append(1) or real(b))
+    block = MinGRUBlock(D, 0)
+    for n, planned in ((257, []), (3, [1])):
+        assert mg._dispatch_block_step(block, torch.zeros(n, D), None, None) is None
+        assert plans == planned
+    assert mg._dispatch_block_step(block, torch.zeros(3, 2, D)[:, 1], None, None) is None
+    assert mg._dispatch_block_step(block.half(), torch.zeros(3, D).half(), None, None) is None
+    assert plans == [1]

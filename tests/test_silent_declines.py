@@ -22,6 +22,7 @@ def _fake(monkeypatch, mode, **impls):
     fake.SCAN_IMPLS = {}
     fake.delta_joined_reason = lambda **kw: None
     fake.angle_joined_reason = lambda *a: None
+    fake.block_step_reason = lambda *a: None
     for name, f in impls.items():
         setattr(fake, name, f)
     monkeypatch.setitem(sys.modules, BACKEND, fake)
