@@ -403,11 +403,13 @@ def _join_backend(x: torch.Tensor, linears, widths, impl: str):
 # layers, 4 to 16 outputs: error against float64 1.4 to 1.6 times larger side by side).
 _JOIN_NARROW = 64
 
-# Multiply-adds of a joined bf16 product from which its backward asks which weights'
-# gradients are wanted.  Forward and one weight's gradient of SignedMinGRU: 374 -> 324 us at
-# 16384 rows of 3 x 1024 outputs (48 Gi; separate layers 339); with half the rows the Python
-# function's host time outweighs the products saved (267 -> 308, separate layers 331).
-_JOIN_ASK_WORK = 1 << 35
+# Multiply-adds of a joined product from which its backward forms only the weights'
+# gradients that are asked for, layer by layer.  Forward and one weight's gradient of
+# SignedMinGRU with 1024 inputs and outputs, us, all weights / the one / separate layers: fp32
+# 4096 rows (12 Gi) 438 / 339 / 357, 2048 rows 307 / 336 / 369; bf16, where a Python function
+# has to stand in for torch's own layer, 16384 rows (48 Gi) 368 / 322 / 345, 8192 rows
+# 274 / 325 / 344: below, the host time outweighs the products saved.
+_JOIN_ASK_WORK = {torch.float32: 1 << 33, torch.bfloat16: 1 << 35}
 
 @functools.lru_cache(maxsize=256)
 def _join_spans(widths: tuple, narrow: int):
@@ -443,13 +445,9 @@ _will_execute = getattr(torch._C, "_will_engine_execute_node", None)
 
 def _asked(node) -> bool:
     """Whether the running backward needs a gradient that goes to ``node``
-    (``needs_input_grad`` of a Python function only says which inputs are trained at all)."""
-    if node is None or _will_execute is None:
-        return node is not None
-    try:
-        return _will_execute(node)
-    except RuntimeError:  # how the engine answers for a leaf that torch.autograd.grad was given
-        return True
+    (``needs_input_grad`` of a Python function only says which inputs are trained at all).
+    Not for a leaf's node: where ``torch.autograd.grad`` was given the leaf the engine raises."""
+    return node is not None and (_will_execute is None or _will_execute(node))
 
 
 class _JoinedLinear(torch.autograd.Function):
@@ -464,9 +462,9 @@ class _JoinedLinear(torch.autograd.Function):
     """
 
     @staticmethod
-    def forward(ctx, x, W, bias, widths):
+    def forward(ctx, x, W, bias, widths, each):
         ctx.save_for_backward(x, W)
-        ctx.widths = widths
+        ctx.widths, ctx.each = widths, each
         return F.linear(x, W, bias)
 
     @staticmethod
@@ -480,19 +478,22 @@ class _JoinedLinear(torch.autograd.Function):
         narrow = _JOIN_NARROW if exact else 0
         if _asked(x_node):
             inputs = _join_spans(ctx.widths, narrow) if exact else [W.shape[0]]
-            for part, w in zip(rows.split(inputs, 1), W.split(inputs)):
-                dx = part @ w if dx is None else dx.addmm_(part, w)
+            for part, w in zip(rows.split_with_sizes(inputs, 1), W.split_with_sizes(inputs)):
+                dx = torch.mm(part, w) if dx is None else dx.addmm_(part, w)
             dx = dx.view(x.shape)
         if _asked(cat):
-            layers = tuple(_asked(node) for node, _ in cat.next_functions)
+            layers = (True,) * len(ctx.widths)
+            if ctx.each:
+                layers = tuple(_asked(node) for node, _ in cat.next_functions)
             spans, asked = _join_weight_spans(ctx.widths, layers, narrow)
             cols, dW = x.reshape(-1, W.shape[1]), torch.empty_like(W)
-            for part, dw, wanted in zip(rows.t().split(spans), dW.split(spans), asked):
+            parts = rows.t().split_with_sizes(spans)
+            for part, dw, wanted in zip(parts, dW.split_with_sizes(spans), asked):
                 if wanted:
                     torch.mm(part, cols, out=dw)
                 else:
                     dw.zero_()
-        return dx, dW, rows.sum(0) if any(map(_asked, biases)) else None, None
+        return dx, dW, rows.sum(0) if any(map(_asked, biases)) else None, None, None
 
 
 def _join_linears(x: torch.Tensor, linears) -> torch.Tensor:
@@ -500,12 +501,14 @@ def _join_linears(x: torch.Tensor, linears) -> torch.Tensor:
     weights, biases = zip(*map(_weight_bias, linears))
     widths = tuple(w.shape[0] for w in weights)
     exact = weights[0].dtype == torch.float32
-    ask = torch.is_grad_enabled() and not torch.is_autocast_enabled() and (
-        exact or x.numel() * sum(widths) >= _JOIN_ASK_WORK)
+    each = x.numel() * sum(widths) >= _JOIN_ASK_WORK[weights[0].dtype]
+    own = torch.is_grad_enabled() and not torch.is_autocast_enabled() and (exact or each)
+    if own and each:
+        weights = [w.view_as(w) for w in weights]
     W, bias = torch.cat(weights), None if biases[0] is None else torch.cat(biases)
-    if ask:
+    if own:
         try:
-            return _JoinedLinear.apply(x, W, bias, widths)
+            return _JoinedLinear.apply(x.view_as(x) if x.is_leaf else x, W, bias, widths, each)
         except RuntimeError:
             pass  # a transform that takes no Python function (forward mode, vmap)
     return F.linear(x, W, bias)

@@ -473,9 +473,9 @@ class _Products(TorchDispatchMode):
 @pytest.mark.parametrize("how", ["grad", "backward"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_joined_linears_form_what_is_asked_for(how, leaf, dtype, monkeypatch):
-    """The input's gradient and each weight's are formed only if they are asked for, the
-    biases' if any of them is: always in fp32, in bf16 past a size (here: any)."""
-    monkeypatch.setattr(mg, "_JOIN_ASK_WORK", 0)
+    """The input's gradient and, past a size (here: any), each weight's are formed only if
+    they are asked for, the biases' if any of them is."""
+    monkeypatch.setitem(mg._JOIN_ASK_WORK, dtype, 0)
     torch.manual_seed(4)
     linears = [nn.Linear(12, n, dtype=dtype) for n in (70, 64, 3, 80)]
     x = torch.randn(18, 12, dtype=dtype, requires_grad=True)
@@ -504,6 +504,17 @@ def test_joined_linears_form_what_is_asked_for(how, leaf, dtype, monkeypatch):
             # magnitude 2, and of their sums.
             torch.testing.assert_close(a, b, **({} if dtype == torch.float32 else
                                                 dict(rtol=2.0**-6, atol=2.0**-6)))
+
+
+def test_small_joined_linears_form_all_weights_or_none():
+    """Below that size the weights' gradients are one joined product if any is asked for."""
+    linears = [nn.Linear(12, n) for n in (70, 64)]
+    x = torch.randn(18, 12, requires_grad=True)
+    for leaves, work in (((linears[1].weight,), 18 * 12 * 134), ((linears[0].bias,), 0)):
+        P = mg._join_linears(x, linears)
+        with _Products() as count:
+            torch.autograd.grad(P, leaves, torch.ones_like(P))
+        assert count.work == work
 
 
 def test_joined_linears_under_transforms():
