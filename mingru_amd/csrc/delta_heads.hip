@@ -15,7 +15,7 @@
 // rows, so the key's norm and the backward's projection are group sums without LDS.
 // HBM-bound copies: neighbouring groups take neighbouring heads of a token, so a wave
 // reads consecutive bytes of P.  At B=8, T=1000, 4 heads of 64, fp32: 14 us each way for
-// 49 and 74 MB; the layer's step, projections included, 1275 -> 609 us.
+// 49 and 74 MB; the layer's step, projections included, 1275 -> 700 to 810 us (host-bound).
 #include "mg_common.h"
 
 #include <type_traits>

@@ -4,8 +4,9 @@
 // Loads are issued unconditionally -- a load under a condition became a branch of its own,
 // with a wait for the register it replaced -- so a step past the sequence end loads the
 // last row again and is made neutral where its value matters.  (linear_scan forward at
-// (16, 4096, 1024) 184 -> 176 us, the MinGRU gates 186 -> 142 us, the signed gates
-// 195 -> 182 us.)  Every offset handed out here is therefore one of a row that exists.
+// (16, 4096, 1024) 184 -> 176 us, the signed gates 195 -> 186 us, the MinGRU gates, with one
+// exponential where there were two, 193 -> 152 us.)  Every offset handed out here is
+// therefore one of a row that exists.
 #pragma once
 
 #include <hip/hip_runtime.h>
