@@ -500,9 +500,12 @@ def _join_linears(x: torch.Tensor, linears) -> torch.Tensor:
     """The outputs of ``linears`` on ``x`` side by side, from one product."""
     weights, biases = zip(*map(_weight_bias, linears))
     widths = tuple(w.shape[0] for w in weights)
-    exact = weights[0].dtype == torch.float32
+    autocast, traced = torch.is_autocast_enabled(), torch.compiler.is_compiling()
+    exact = weights[0].dtype == torch.float32 and not autocast
+    if exact and traced:  # no engine to ask, and no sums longer than the layers' own either
+        return torch.cat([F.linear(x, w, b) for w, b in zip(weights, biases)], -1)
     each = x.numel() * sum(widths) >= _JOIN_ASK_WORK[weights[0].dtype]
-    own = torch.is_grad_enabled() and not torch.is_autocast_enabled() and (exact or each)
+    own = torch.is_grad_enabled() and not (autocast or traced) and (exact or each)
     if own and each:
         weights = [w.view_as(w) for w in weights]
     W, bias = torch.cat(weights), None if biases[0] is None else torch.cat(biases)

@@ -517,6 +517,42 @@ def test_small_joined_linears_form_all_weights_or_none():
         assert count.work == work
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_joined_linears_compile(dtype, monkeypatch):
+    """Traced, where the engine can't be asked, the products are torch's own."""
+    monkeypatch.setitem(mg._JOIN_ASK_WORK, dtype, 0)
+    torch.manual_seed(5)
+    linears = [nn.Linear(6, n, dtype=dtype) for n in (66, 2)]
+    x = torch.randn(2, 4, 6, dtype=dtype, requires_grad=True)
+    leaves = [x, *(p for m in linears for p in m.parameters())]
+    got = torch.compile(lambda x: mg._join_linears(x, linears), backend="aot_eager")(x)
+    want = torch.cat([m(x) for m in linears], -1)
+    g = torch.randn_like(want)
+    for a, b in zip([got, *torch.autograd.grad(got, leaves, g)],
+                    [want, *torch.autograd.grad(want, leaves, g)]):
+        torch.testing.assert_close(a, b, **({} if dtype == torch.float32 else
+                                            dict(rtol=2.0**-6, atol=2.0**-6)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("build", [lambda: MinGRU(64, 64), lambda: GivensMinGRU(64, 64),
+                                   lambda: DeltaMinGRU(64, 64, n_heads=2)])
+def test_joined_layers_compile(cuda, build, monkeypatch):
+    """A compiled fp32 layer equals the eager one."""
+    monkeypatch.setenv("MINGRU_SCAN", "hip")
+    print("[gpu] compiled joined layer", flush=True)
+    torch.manual_seed(6)
+    m = build().to(cuda)
+    x = torch.randn(2, 200, 64, device=cuda, requires_grad=True)
+    torch._dynamo.reset()
+    y, want = torch.compile(m, backend="aot_eager")(x), m(x)
+    g = torch.randn_like(want)
+    leaves = [x, *m.parameters()]
+    for a, b in zip([y, *torch.autograd.grad(y, leaves, g)],
+                    [want, *torch.autograd.grad(want, leaves, g)]):
+        assert _off(a, b) <= 2e-5
+
+
 def test_joined_linears_under_transforms():
     """Forward mode and vmap, which take no Python function, take the plain product."""
     torch.manual_seed(3)
