@@ -340,6 +340,15 @@ int mg_delta_heads_bwd(const void* K, const void* beta, const float* nrm, const 
                        const void* dK, const void* dV, const void* dbeta, void* dP, int64_t B,
                        int64_t T, int H, int nh, int dk, int dv, int dtype, mg_stream_t stream);
 
+/* ---- column sums ------------------------------------------------------------------
+ * out (N) = the sums over the rows of x (rows, N), both in dtype (0 fp32, 1 bf16), summed in
+ * fp32 in a fixed order.  No reference kernel: torch's sum, without its cleared counters, for
+ * bias gradients under graph capture.  rows <= 2^36, N <= 2^24; the workspace needs no
+ * initialisation. */
+size_t mg_column_sums_workspace_bytes(int64_t rows, int64_t N);
+int mg_column_sums(const void* x, void* out, int64_t rows, int64_t N, int dtype, void* ws,
+                   size_t ws_bytes, mg_stream_t stream);
+
 /* ---- elementwise scans on bf16 tensors --------------------------------------------
  * The scans above with bf16 tensors (void*), computed in fp32.  No reference
  * kernels: the reference casts to fp32 around its fp32 kernels

@@ -109,6 +109,8 @@ _SIGNATURES = {
     ),
     "mg_delta_heads_fwd": (_I32, [_P] * 6 + [_I64, _I64] + [_I32] * 5 + [_P]),
     "mg_delta_heads_bwd": (_I32, [_P] * 8 + [_I64, _I64] + [_I32] * 5 + [_P]),
+    "mg_column_sums_workspace_bytes": (_SZ, [_I64, _I64]),
+    "mg_column_sums": (_I32, [_P, _P, _I64, _I64, _I32, _P, _SZ, _P]),
     "mg_delta_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I32, _I32, _I32, _I32]),
     "mg_delta_state_bytes": (_SZ, [_I64, _I64, _I64, _I32, _I32, _I32, _I32]),
     "mg_delta_fwd": (

@@ -45,6 +45,7 @@ __all__ = [
     "angle_joined_reason",
     "delta_heads_impl",
     "delta_joined_reason",
+    "column_sums",
     "block_step_impl",
     "block_step_reason",
     "workspace_errors",
@@ -1572,6 +1573,20 @@ def delta_scan_impl(Q, K, V, beta, H0, *, chunk_size: int):
         return Q.new_zeros(Q.shape[:3] + (V.shape[-1],)), H0.clone()
     return _funnel("DeltaMinGRU chunked-WY", _DeltaScanFn.apply, Q, K, V, beta, H0,
                    _delta_tile_chunk(K.shape[3], chunk_size))
+
+
+def column_sums(x: torch.Tensor) -> torch.Tensor:
+    """``x.sum(0)`` of an (rows, N) fp32 or bf16 GPU tensor, safe in a graph that is replayed
+    (csrc/column_sums.hip).  Not differentiable."""
+    if x.ndim != 2 or x.numel() == 0 or x.dtype not in (torch.float32, torch.bfloat16):
+        raise ScanFallback(f"column sums of {tuple(x.shape)} {x.dtype}")
+    x = x.contiguous()
+    rows, N = x.shape
+    out = torch.empty(N, dtype=x.dtype, device=x.device)
+    ws = _workspace(_size("mg_column_sums_workspace_bytes", rows, N), x.device)
+    _call("mg_column_sums", _ptr(x), _ptr(out), rows, N, int(x.dtype == torch.bfloat16), _ptr(ws),
+          ws.numel(), _stream(x))
+    return out
 
 
 class _DeltaHeadsFn(torch.autograd.Function):

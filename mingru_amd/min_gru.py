@@ -371,8 +371,13 @@ def _join_backend(x: torch.Tensor, linears, widths, impl: str):
         return None
     if torch.nn.modules.module._has_any_global_hook():
         return None
-    if linears[0].weight.dtype not in (torch.float32, torch.bfloat16) or (
-        torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") != torch.bfloat16
+    if linears[0].weight.dtype not in (torch.float32, torch.bfloat16):
+        return None
+    # Under autocast the joined product is torch's own layer, whose bias gradient does not
+    # replay at every width (_bias_gradient).
+    if torch.is_autocast_enabled() and (
+        torch.get_autocast_dtype("cuda") != torch.bfloat16
+        or (torch.is_grad_enabled() and _capturing(x))
     ):
         return None
     if len(linears) != len(widths):
@@ -450,6 +455,19 @@ def _asked(node) -> bool:
     return node is not None and (_will_execute is None or _will_execute(node))
 
 
+def _capturing(x: torch.Tensor) -> bool:
+    return x.is_cuda and torch.cuda.is_current_stream_capturing()
+
+
+def _bias_gradient(rows: torch.Tensor) -> torch.Tensor:
+    """``rows.sum(0)``.  Not by torch where it is captured: its sum clears counters with a
+    memset, which has left them as they were on replays of the graph after the first."""
+    if _capturing(rows):
+        from mingru_amd import hip_scans
+        return hip_scans.column_sums(rows)
+    return rows.sum(0)
+
+
 class _JoinedLinear(torch.autograd.Function):
     """Layers of ``widths`` outputs side by side, ``x W^T + bias``: one product forward, and a
     backward that forms only the gradients that are asked for, in fp32 in sums no longer than
@@ -493,7 +511,7 @@ class _JoinedLinear(torch.autograd.Function):
                     torch.mm(part, cols, out=dw)
                 else:
                     dw.zero_()
-        return dx, dW, rows.sum(0) if any(map(_asked, biases)) else None, None, None
+        return dx, dW, _bias_gradient(rows) if any(map(_asked, biases)) else None, None, None
 
 
 def _join_linears(x: torch.Tensor, linears) -> torch.Tensor:
@@ -505,7 +523,8 @@ def _join_linears(x: torch.Tensor, linears) -> torch.Tensor:
     if exact and traced:  # no engine to ask, and no sums longer than the layers' own either
         return torch.cat([F.linear(x, w, b) for w, b in zip(weights, biases)], -1)
     each = x.numel() * sum(widths) >= _JOIN_ASK_WORK[weights[0].dtype]
-    own = torch.is_grad_enabled() and not (autocast or traced) and (exact or each)
+    own = torch.is_grad_enabled() and not (autocast or traced) and (
+        exact or each or _capturing(x))
     if own and each:
         weights = [w.view_as(w) for w in weights]
     W, bias = torch.cat(weights), None if biases[0] is None else torch.cat(biases)

@@ -11,7 +11,8 @@ synchronisations between the replays, and checks every replay against eager.
 import pytest
 import torch
 
-from mingru_amd import hip_scans, linear_scan, parallel_scan_log
+from mingru_amd import (DeltaMinGRU, GivensMinGRU, MinGRU, SignedMinGRU, hip_scans,
+                        linear_scan, parallel_scan_log)
 from mingru_amd.min_gru import _dispatch_mingru_gate_scan
 
 pytestmark = pytest.mark.gpu
@@ -147,3 +148,63 @@ def test_log_scan_fwd_bwd_graph_replays(cuda):
         torch.cuda.synchronize()
         for name, x, r in zip(("h", "dlc", "dlv"), out, ref):
             assert torch.allclose(x, r, rtol=1e-5, atol=1e-6), f"replay {rep}: {name}"
+
+
+# Joined widths of 772, 896 and 640 columns, at which torch's own sum over the rows does not
+# replay, and 768, at which it does.
+JOINED = [
+    (lambda: DeltaMinGRU(256, 256, n_heads=4), torch.float32, False),
+    (lambda: DeltaMinGRU(256, 256, n_heads=4), torch.bfloat16, False),
+    (lambda: GivensMinGRU(256, 256), torch.float32, False),
+    (lambda: MinGRU(256, 320), torch.bfloat16, True),
+    (lambda: SignedMinGRU(256, 256), torch.bfloat16, False),
+]
+
+
+@pytest.mark.parametrize("case", range(len(JOINED)))
+def test_joined_layer_training_replays(cuda, case):
+    """A captured training pass of a layer with joined projections, every gradient."""
+    build, dtype, autocast = JOINED[case]
+    print(f"[gpu] graph: joined layer case={case}", flush=True)
+    torch.manual_seed(case)
+    m = build().to(cuda, torch.float32 if autocast else dtype)
+    x = torch.randn(4, 1000, 256, device=cuda, dtype=next(m.parameters()).dtype,
+                    requires_grad=True)
+    leaves = [x, *m.parameters()]
+
+    def step():
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast, cache_enabled=False):
+            y = m(x)
+        return [y.detach(), *torch.autograd.grad(y, leaves, torch.ones_like(y) + y.detach())]
+
+    g, static = _capture(step, ())
+    for rep in range(4):
+        with torch.no_grad():
+            x.copy_(torch.randn_like(x))
+        g.replay()
+        eager = step()
+        torch.cuda.synchronize()
+        for i, (a, b) in enumerate(zip(static, eager)):
+            off = ((a.double() - b.double()).norm() / b.double().norm()).item()
+            # The same kernels but for the bias sums' order; bf16 outputs round it.
+            bound = 2e-5 if a.dtype == torch.float32 and not autocast else 2e-2
+            assert off <= bound, f"replay {rep}, output {i}: {off:.2e}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,N", [(1, 1), (3, 63), (64, 64), (65, 65), (255, 130), (1000, 772),
+                                    (16385, 96), (40001, 7)])
+def test_column_sums(cuda, rows, N, dtype):
+    """Against float64: additions in chains of a chunk's rows / 16 and of chunks / 4, 2^-24 of
+    the absolute sum each, and the output's rounding (bf16: 2^-8)."""
+    print(f"[gpu] column sums {rows}x{N} {dtype}", flush=True)
+    gen = torch.Generator(device=cuda).manual_seed(rows)
+    x = torch.randn(rows, N, device=cuda, generator=gen).to(dtype)
+    got = hip_scans.column_sums(x)
+    want, size = x.double().sum(0), x.double().abs().sum(0)
+    chunks = min(256, -(-rows // 64))
+    depth = -(-rows // chunks) / 16 + 4 + chunks / 4 + 6
+    bound = depth * 2.0**-24 * size + (2.0**-8 if dtype == torch.bfloat16 else 0.0) * want.abs()
+    assert got.dtype == dtype and got.shape == (N,)
+    assert ((got.double() - want).abs() <= bound + 1e-30).all()
+    torch.testing.assert_close(hip_scans.column_sums(x.t().contiguous().t()), got, rtol=0, atol=0)

@@ -500,8 +500,8 @@ def test_joined_linears_form_what_is_asked_for(how, leaf, dtype, monkeypatch):
                 got = [t.grad for t in leaves]
         assert (count.work, count.sums) == (work, sums)
         for a, b in zip(got, torch.autograd.grad(want, leaves, g, retain_graph=True)):
-            # bf16: half a unit (2^-9) for each of the separate input gradient's four parts, of
-            # magnitude 2, and of their sums.
+            # bf16: a rounding (2^-8) for each of the separate input gradient's four parts, of
+            # magnitude 2, and for their sums.
             torch.testing.assert_close(a, b, **({} if dtype == torch.float32 else
                                                 dict(rtol=2.0**-6, atol=2.0**-6)))
 
